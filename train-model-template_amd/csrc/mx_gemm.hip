@@ -4,14 +4,21 @@
 // Replaces torch._scaled_mm (cuBLAS block-scaled GEMM) at /root/reference/scripts/fused_mlp.py:279, :283, :309,
 // :329 and the addmm_ epilogues at :284 and :331.
 //
-// Tiling: a workgroup computes a 256 (M) x 128 (N) tile with four waves, two workgroups per CU (kNW = 1;
-// layout bit MXFP8_GEMM_WIDE selects the 8-wave 256 x 256 shape, kNW = 2, one workgroup per CU), in K steps
-// of 64 (two scale blocks).  Measured on the four MLP GEMMs (T=10752, d=2048, f=6144): 845-858 us at
-// kNW = 1 against 873-908 us at kNW = 2 with its best tail split.  Each wave
-// holds a 64 (M) x 128 (N) sub-tile as a 2 x 4 grid of 32 x 32 MFMA tiles (128 accumulators per lane), so two
-// waves share each SIMD; with two independent workgroups per CU one workgroup's pipeline fill, barrier waits
-// and epilogue overlap the other's matrix work.  The matrix instruction takes the weight (B) fragment as its
-// first operand, so each lane's accumulators cover one output row m and 16 columns n in runs of 4.
+// Tiling: a workgroup computes a 256 (M) x 128 (N) tile with four waves, two workgroups per CU (Tall; layout bit
+// MXFP8_GEMM_WIDE selects the 8-wave 256 x 256 shape, Wide, one workgroup per CU), in K steps of 64 (two scale
+// blocks).  Each wave holds a 64 (M) x 128 (N) sub-tile as a 2 x 4 grid of 32 x 32 MFMA tiles (128 accumulators
+// per lane), so two waves share each SIMD; with two independent workgroups per CU one workgroup's pipeline fill,
+// barrier waits and epilogue overlap the other's matrix work.  The matrix instruction takes the weight (B)
+// fragment as its first operand, so each lane's accumulators cover one output row m and 16 columns n in runs of 4.
+//
+// Order inside a K step: a wave issues its instructions in order, so whatever stands between two MFMAs runs while
+// the first one executes.  The step's DMAs and fragment reads are spread evenly over its MFMAs, and the DMAs take
+// a wave-uniform base with a 32-bit lane offset (no 64-bit address arithmetic on the vector pipe).  Left to the
+// compiler the DMAs stood in one block, and the fragment reads behind them in another, right before the wait for
+// them at the step's end.  us per launch at T = 10752, before -> now (d_model 2048, d_ffn 6144; two builds in one
+// process, alternating): down 121 -> 112, dx 230 -> 211, dh 131 -> 122, gate|up (no epilogue) 253 -> 243; a lone
+// workgroup per CU (T = 256, K = 12288) 66 -> 57; Wide at T = 142336: dx 2692 -> 2568, down 1406 -> 1366.  All
+// outputs are bit-identical.
 //
 // What bounds it (rocprofv3 counters on the MLP GEMMs): the CU's vector-memory path that carries the
 // operand DMA (TA / TD busy 65-89% of the kernel, TD waiting on L1/L2 data about 45% of the time) while the
@@ -26,10 +33,10 @@
 // bit-identical.
 //
 // Operand staging: global memory goes straight into LDS with global_load_lds_dwordx4 (no VGPR round trip)
-// through a ring of 3 stages of 26 KB (kNW = 2: 4 of 34 KB): A codes 256 x 64 B, B codes 128 x 64 B, and the
-// 128-row blocked scale tiles of each operand for the current 128-wide K tile.  Every wave issues the same
-// number of DMA instructions per stage (1 KB code slices of A and of B plus a scale tile or a duplicate), so a
-// fixed vmcnt bounds the wait for a stage while the later ones stay in flight.  Lane i of a DMA lands at
+// through a ring of 3 stages of 26 KB (Wide: 4 of 34 KB): A codes 256 x 64 B, B codes 128 x 64 B, and the
+// 128-row blocked scale tiles of each operand for the current 128-wide K tile, these in 256-byte pieces
+// (global_load_lds_dword) so that every wave issues the same DMAs and none is a filler: a fixed vmcnt bounds the
+// wait for a stage while the later ones stay in flight.  Lane i of a DMA lands at
 // base + 16 i; a row's 16-byte chunk c is stored at chunk c ^ ((row >> 2) & 3): the gfx950 LDS serves a
 // ds_read_b128 16 lanes (16 consecutive rows, same chunk) at a time over 64 banks, and with 64-byte rows
 // rows r, r+4, r+8, r+12 share bank groups unless their chunks differ (measured: 48% bank-conflict cycles
@@ -38,7 +45,7 @@
 // groups' scales for one 128-wide K tile; a lane shifts its word by 8 * (lane / 32) so that op_sel 0 / 2
 // selects block 2P + lane/32 of the current half-tile P.
 // Work order: a 1-D grid in which workgroup i runs on XCD i % 8 (the dispatcher's round robin).  Tiles are
-// numbered in groups of kGroupM M-tiles (M fastest inside a group) and each XCD takes a contiguous range of
+// numbered in groups of 1024 rows of M-tiles (M fastest inside a group) and each XCD takes a contiguous range of
 // that order, so the tiles resident on one XCD share A and B panels in its L2.  With the 8-wave shape, when
 // the last wave of tiles would fill at most half of the CUs, those tail tiles are split along K into `parts`
 // pieces run as separate workgroups after the full tiles; each piece writes its fp32 accumulators to the
@@ -66,30 +73,35 @@ using namespace mxk;
 
 namespace {
 
-constexpr int kBM = 256, kBK = 64;
-constexpr int kCodeBytes = kBM * kBK;  // A codes per stage: 16 KB
-constexpr int kGroupM = 4;
+constexpr int kBK = 64;
 constexpr int kMaxParts = 4;
 // Workspace layout: arrival counters at a fixed place (so every shape finds its own counters at zero, each
 // launch resets those it used), fp32 partial tiles after them.
 constexpr int64_t kCounterBytes = 4096;
 constexpr int kMaxSplitTiles = (int)(kCounterBytes / 4);
 
-// Workgroup shapes.  kNW = 2: 8 waves, 256 x 256 tile, 4-stage ring of 34 KB (one workgroup per CU).
-// kNW = 1: 4 waves, 256 x 128 tile, 3-stage ring of 26 KB (two workgroups per CU, whose barriers are
-// independent, so one workgroup's MFMAs fill the other's waits).  Every wave computes a 64 (M) x 128 (N)
-// sub-tile either way.
-template <int kNW>
+// Workgroup shapes: a grid of kWM x kWN waves, each wave computing kMB x kNB blocks of 32 x 32, over a ring of
+// kStages_ stages.
+template <int kMB_, int kNB_, int kWM_, int kWN_, int kKS_, int kStages_>
 struct Shape {
-  static constexpr int kWaves = 4 * kNW, kThreads = 64 * kWaves, kBN = 128 * kNW;
-  static constexpr int kStages = kNW == 2 ? 4 : 3;
-  static constexpr int kOffA = 0, kOffB = kCodeBytes, kOffSA = kCodeBytes + kBN * kBK, kOffSB = kOffSA + 1024;
-  static constexpr int kStageBytes = kOffSB + 1024;
-  // DMA per wave and stage: kSA 1 KB slices of A, kSB of B, and one more (A's or B's scale tiles, or a
-  // repeat of the wave's last B slice), so a fixed vmcnt bounds every wait.
-  static constexpr int kSA = 16 / kWaves, kSB = (kBN / 16) / kWaves, kDma = kSA + kSB + 1;
+  static constexpr int kMB = kMB_, kNB = kNB_, kWM = kWM_, kWN = kWN_, kKS = kKS_, kStages = kStages_;
+  static constexpr int kWaves = kWM * kWN, kThreads = 64 * kWaves;
+  static constexpr int kBM = 32 * kMB * kWM, kBN = 32 * kNB * kWN;
+  static constexpr int kGroupM = 1024 / kBM;  // M-tiles of a tile group (1024 rows)
+  static constexpr int kTilesA = (kBM + 127) / 128, kTilesB = (kBN + 127) / 128;  // 128-row scale tiles
+  static constexpr int kSliceA = kBM * kBK, kSliceB = kBN * kBK;  // codes of one 64-wide K slice
+  static constexpr int kOffA = 0, kOffB = kKS * kSliceA, kOffS = kOffB + kKS * kSliceB;
+  static constexpr int kOffSB = kOffS + kTilesA * 512;
+  static constexpr int kStageBytes = kOffS + (kTilesA + kTilesB) * 512;
+  // DMA per wave and stage: kSA 1 KB slices of A, kSB of B, and kSS 256-byte pieces of the scale tiles (a wave
+  // past the last piece repeats it: same source, same destination), so a fixed vmcnt bounds every wait.
+  static constexpr int kSA = (kBM / 16) / kWaves, kSB = (kBN / 16) / kWaves;
+  static constexpr int kPieces = (kTilesA + kTilesB) * 2, kSS = (kPieces + kWaves - 1) / kWaves;
+  static constexpr int kDma = kKS * (kSA + kSB) + kSS;
   static constexpr int64_t kPartBytes = (int64_t)kBM * kBN * 4;  // fp32 partial tile
 };
+using Tall = Shape<2, 4, 4, 1, 1, 3>;   // 256 x 128, 4 waves, ring 78 KB: two workgroups per CU
+using Wide = Shape<2, 4, 4, 2, 1, 4>;   // 256 x 256, 8 waves, ring 136 KB: one workgroup per CU
 
 struct Lora {
   const uint16_t* p;  // [M, r] bf16
@@ -153,7 +165,7 @@ constexpr int kEpiPlain = 0, kEpiSwiGluFwd = 1, kEpiSwiGluBwd = 2;
 constexpr int kBwdTrBytes = 3 * 32 * kTrLd * 2;
 constexpr int kBwdDbOff = 4 * kBwdTrBytes, kBwdDbBytes = 4 * 3 * 512 * 4;
 constexpr int kBwdWOff = kBwdDbOff + kBwdDbBytes, kBwdWBytes = 6 * 128 * 16 * 2;
-static_assert(kBwdWOff + kBwdWBytes <= Shape<1>::kStages * Shape<1>::kStageBytes, "backward epilogue LDS");
+static_assert(kBwdWOff + kBwdWBytes <= Tall::kStages * Tall::kStageBytes, "backward epilogue LDS");
 static_assert(3 * 32 * 16 * 4 <= kBwdTrBytes, "dB exchange fits a wave's transpose tiles");
 
 // Output columns in up to four segments, each its own row-major matrix: columns [col0[k], col0[k + 1]) of the
@@ -180,6 +192,7 @@ struct Plan {
   int* cnt;          // [nsplit] arrival counters (zero between launches)
 };
 
+template <int kGroupM>
 __device__ __forceinline__ void tile_coords(int t, int tm, int tn, int& mt, int& nt) {
   const int g = t / (kGroupM * tn), r = t - g * (kGroupM * tn);
   const int rows = min(kGroupM, tm - g * kGroupM);
@@ -191,14 +204,29 @@ __device__ __forceinline__ void tile_coords(int t, int tm, int tn, int& mt, int&
 // the rank-16, 32 or 48 LoRA epilogue, the dx GEMMs of the fused MLP (r = 32 at r = 16 adapters) and of the
 // grouped linears (q|k|v: 48, o_proj: 16).  At configuration 3 each has 672 tiles, 1.3 rounds of the workgroup
 // slots.  Other instances do not compile the reduction.
-template <int kR, int kNW, int kEpi>
-constexpr bool kFoldTn = (kR == 16 || kR == 32 || kR == 48) && kNW == 1 && kEpi == 0;
+template <int kR, class S, int kEpi>
+constexpr bool kFoldTn = (kR == 16 || kR == 32 || kR == 48) && S::kThreads == 256 && kEpi == 0;
 // The instance whose epilogue operand P can be summed in its own launch (mxfp8_gemm_nt_sum): the plain 4-wave GEMM
 // with the rank-16 epilogue, the fused MLP's down GEMM at r = 16.
-template <int kR, int kNW, int kEpi>
-constexpr bool kFoldSum = kR == 16 && kNW == 1 && kEpi == 0;
-static_assert(tn_batch_lds_elems<true>() * 2 <= 3 * 26 * 1024,
-              "the folded token reduction borrows the 4-wave ring's LDS");
+template <int kR, class S, int kEpi>
+constexpr bool kFoldSum = kR == 16 && S::kThreads == 256 && kEpi == 0;
+template <class S>
+constexpr bool kTnFits = tn_batch_lds_elems<true>() * 2 <= S::kStages * S::kStageBytes;
+static_assert(kTnFits<Tall>, "the folded token reduction borrows the 4-wave ring's LDS");
+
+// n scale words (4-byte aligned to their count) from LDS
+template <int n>
+__device__ __forceinline__ void read_words(const uint8_t* p, uint32_t* w) {
+  if constexpr (n == 4) {
+    const uint4 v = *reinterpret_cast<const uint4*>(p);
+    w[0] = v.x; w[1] = v.y; w[2] = v.z; w[3] = v.w;
+  } else if constexpr (n == 2) {
+    const uint2 v = *reinterpret_cast<const uint2*>(p);
+    w[0] = v.x; w[1] = v.y;
+  } else {
+    w[0] = *reinterpret_cast<const uint32_t*>(p);
+  }
+}
 
 // 32 bytes of one operand row for the stage's 64-wide K step: chunk c0 (k 16*(l/32)..) and c0 + 2 (k 32 + ..)
 __device__ __forceinline__ v8i frag(const uint8_t* base, int row, int c0, int sw) {
@@ -210,21 +238,22 @@ __device__ __forceinline__ v8i frag(const uint8_t* base, int row, int c0, int sw
   return r;
 }
 
-template <int kR, int kNW, int kEpi>
-__global__ __launch_bounds__(Shape<kNW>::kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_kernel(
+template <int kR, class S, int kEpi>
+__global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_kernel(
     const uint8_t* __restrict__ A, const uint8_t* __restrict__ SA, int64_t lda, const uint8_t* __restrict__ B,
     const uint8_t* __restrict__ SB, int64_t ldb, int M, int N, int K, CSeg cseg, Lora lora, Plan plan, int tiled,
     SwEpi swe, SwBwd swb, const TnBatch tnb, const PreSum pre) {
-  using S = Shape<kNW>;
+  constexpr int kMB = S::kMB, kNB = S::kNB, kBM = S::kBM;
   __shared__ __attribute__((aligned(16))) uint8_t lds[S::kStages * S::kStageBytes];
   __shared__ int arrived;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
-  const int wn = wave >> 2, wm = wave & 3;  // compute sub-tile: n rows wn*128 + [0,128), m rows wm*64 + [0,64)
+  // compute sub-tile: n rows wn * 32 kNB + [0, 32 kNB), m rows wm * 32 kMB + [0, 32 kMB)
+  const int wn = wave / S::kWM, wm = wave % S::kWM;
 
   // ---- workgroups before the tiles: the sum of the epilogue operand P (mxfp8_gemm_nt_sum, presum_device.h)
   int bid = blockIdx.x;
-  if constexpr (kFoldSum<kR, kNW, kEpi>) {
+  if constexpr (kFoldSum<kR, S, kEpi>) {
     if (bid < pre.blocks) {
       presum_block(pre, bid);
       return;
@@ -235,7 +264,7 @@ __global__ __launch_bounds__(Shape<kNW>::kThreads) __attribute__((amdgpu_waves_p
   // ---- workgroups past the tiles: the folded token reductions (mxfp8_gemm_nt_tn), in the ring's LDS.  They are
   // numbered after every tile, so the dispatcher starts them only once each tile has started, in the slots the
   // last round of tiles leaves free.
-  if constexpr (kFoldTn<kR, kNW, kEpi>) {
+  if constexpr (kFoldTn<kR, S, kEpi>) {
     const int first = 8 * (plan.per_full + plan.per_split);
     if (bid >= first) {
       uint16_t* tl = reinterpret_cast<uint16_t*>(lds);
@@ -264,7 +293,7 @@ __global__ __launch_bounds__(Shape<kNW>::kThreads) __attribute__((amdgpu_waves_p
     }
   }
   int mt_, nt_;
-  tile_coords(tile, plan.tm, plan.tn, mt_, nt_);
+  tile_coords<S::kGroupM>(tile, plan.tm, plan.tn, mt_, nt_);
   const int m0 = mt_ * kBM, n0 = nt_ * S::kBN;
   const int nkt = K / 128;
 
@@ -292,71 +321,78 @@ __global__ __launch_bounds__(Shape<kNW>::kThreads) __attribute__((amdgpu_waves_p
   for (int j = 0; j < S::kSA; ++j) goa[j] = slice_off(a_tiled, m0, M, lda, (wave * S::kSA + j) * 16);
 #pragma unroll
   for (int j = 0; j < S::kSB; ++j) gob[j] = slice_off(b_tiled, n0, N, ldb, (wave * S::kSB + j) * 16);
-  // Last DMA of the stage, without divergence: wave 0 copies A's two 128-row scale tiles, wave 1 B's
-  // scale tile(s) (1 KB, lane -> tile lane / 32, bytes (lane % 32) * 16 of it; for a 128-row B tile the
-  // upper half holds the next tile's, unused); the other waves repeat their last B slice (same source, same
-  // destination: a harmless duplicate).
-  const bool scl = wave < 2;
-  const int sR0 = wave == 0 ? m0 : n0, sRn = wave == 0 ? M : N;
-  const int stile = min((sR0 >> 7) + (lane >> 5), (sRn - 1) >> 7);
-  const uint8_t* sgp = (wave == 0 ? SA : SB) + (int64_t)stile * nkt * 512 + (lane & 31) * 16;
+  // The stage's scale tiles (kTilesA of A, kTilesB of B; 512 bytes each, for the K step's 128-wide K tile) in pieces
+  // of 256 bytes, 4 bytes a lane, kSS pieces a wave, so every wave issues the same DMAs.
+  const uint8_t* gsp[S::kSS];
+  int dma_s_off[S::kSS];
+#pragma unroll
+  for (int j = 0; j < S::kSS; ++j) {
+    const int pc = min(wave * S::kSS + j, S::kPieces - 1), ti = pc >> 1;  // wave-uniform
+    const bool is_a = ti < S::kTilesA;
+    const int rt = is_a ? min((m0 >> 7) + ti, (M - 1) >> 7) : min((n0 >> 7) + ti - S::kTilesA, (N - 1) >> 7);
+    gsp[j] = (is_a ? SA : SB) + (int64_t)rt * nkt * 512 + (pc & 1) * 256;
+    dma_s_off[j] = S::kOffS + pc * 256;
+  }
   const int dma_a_off = S::kOffA + wave * S::kSA * 1024, dma_b_off = S::kOffB + wave * S::kSB * 1024;
-  const int dma_x_off = wave == 0 ? S::kOffSA : wave == 1 ? S::kOffSB : dma_b_off + (S::kSB - 1) * 1024;
 
   const uint32_t lds0 = lds_addr(lds);
-  const int last = s_end - 1;
-  auto issue_to = [&](int s, int slot) {  // DMA stage s into ring slot `slot`
+  // Stage s: kKS 64-wide K slices, the scale tiles of the 128-wide K tile they lie in.
+  const int s0 = s_begin / S::kKS, last = s_end / S::kKS - 1;
+  auto dma = [&](int s, int slot, int d) {  // DMA d of stage s into ring slot `slot` (d a constant once unrolled)
     const uint32_t st = lds0 + slot * S::kStageBytes;
-    const uint8_t* pa = ga + s * sa_stride;
-    const uint8_t* pb = gb + s * sb_stride;
+    constexpr int nA = S::kKS * S::kSA, nB = S::kKS * S::kSB;
+    if (d < nA) {
+      const int k = d / S::kSA, j = d % S::kSA;
+      dma16_at(ga + (s * S::kKS + k) * sa_stride, goa[j], st + dma_a_off + k * S::kSliceA + j * 1024);
+    } else if (d < nA + nB) {
+      const int k = (d - nA) / S::kSB, j = (d - nA) % S::kSB;
+      dma16_at(gb + (s * S::kKS + k) * sb_stride, gob[j], st + dma_b_off + k * S::kSliceB + j * 1024);
+    } else {
+      dma4_at(gsp[d - nA - nB] + (S::kKS == 2 ? s : s >> 1) * 512, lane * 4, st + dma_s_off[d - nA - nB]);
+    }
+  };
+  auto issue_to = [&](int s, int slot) {
 #pragma unroll
-    for (int j = 0; j < S::kSA; ++j) dma16(pa + goa[j], st + dma_a_off + j * 1024);
-#pragma unroll
-    for (int j = 0; j < S::kSB; ++j) dma16(pb + gob[j], st + dma_b_off + j * 1024);
-    dma16(scl ? sgp + (s >> 1) * 512 : pb + gob[S::kSB - 1], st + dma_x_off);
+    for (int d = 0; d < S::kDma; ++d) dma(s, slot, d);
   };
 
-  v16f acc[4][2];
+  v16f acc[kNB][kMB];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    acc[i][0] = v16f{};
-    acc[i][1] = v16f{};
-  }
+  for (int i = 0; i < kNB; ++i)
+#pragma unroll
+    for (int j = 0; j < kMB; ++j) acc[i][j] = v16f{};
 
   const int sshift = (lane >> 5) * 8;
   const int sw = (lane >> 2) & 3;  // swizzle of rows base + lane % 32 (base a multiple of 32)
   const int c0 = lane >> 5;
+  // the wave's first row / column inside the workgroup's 128-row scale tiles
+  const int rwa = (kBM < 128 ? m0 & 127 : 0) + wm * 32 * kMB, rwb = (S::kBN < 128 ? n0 & 127 : 0) + wn * 32 * kNB;
+  const int sa_off = S::kOffS + (rwa >> 7) * 512 + (lane & 31) * 16 + ((rwa >> 5) & 3) * 4;
+  const int sb_off = S::kOffSB + (rwb >> 7) * 512 + (lane & 31) * 16 + ((rwb >> 5) & 3) * 4;
   struct Frags {
-    v8i a0, a1, b0, b1, b2, b3;
-    uint2 sa;
-    uint4 sb;
+    v8i a[S::kKS][kMB], b[S::kKS][kNB];
+    uint32_t sa[kMB], sb[kNB];
   };
-  auto read = [&](int slot, Frags& f) {
+  // a stage's fragments, one at a time: its scale words, then per K slice kMB of A and kNB of B
+  constexpr int kReads = S::kKS * (kMB + kNB), kMfma = S::kKS * kMB * kNB;
+  auto read_scales = [&](int slot, Frags& f) {
     const uint8_t* st = lds + slot * S::kStageBytes;
-    f.sa = *reinterpret_cast<const uint2*>(st + S::kOffSA + (wm >> 1) * 512 + (lane & 31) * 16 + (wm & 1) * 8);
-    f.sb = *reinterpret_cast<const uint4*>(st + S::kOffSB + wn * 512 + (lane & 31) * 16);
-    const uint8_t* la = st + S::kOffA;
-    const uint8_t* lb = st + S::kOffB;
-    f.a0 = frag(la, wm * 64 + (lane & 31), c0, sw);
-    f.a1 = frag(la, wm * 64 + 32 + (lane & 31), c0, sw);
-    f.b0 = frag(lb, wn * 128 + (lane & 31), c0, sw);
-    f.b1 = frag(lb, wn * 128 + 32 + (lane & 31), c0, sw);
-    f.b2 = frag(lb, wn * 128 + 64 + (lane & 31), c0, sw);
-    f.b3 = frag(lb, wn * 128 + 96 + (lane & 31), c0, sw);
+    read_words<kMB>(st + sa_off, f.sa);
+    read_words<kNB>(st + sb_off, f.sb);
   };
-  auto mma = [&](const Frags& f, auto pc) {
-    constexpr int P = decltype(pc)::value;  // half of the 128-wide K tile: blocks 2P, 2P + 1
-    const int sa0 = (int)(f.sa.x >> sshift), sa1 = (int)(f.sa.y >> sshift);
-    const int sb0 = (int)(f.sb.x >> sshift), sb1 = (int)(f.sb.y >> sshift);
-    const int sb2 = (int)(f.sb.z >> sshift), sb3 = (int)(f.sb.w >> sshift);
-    acc[0][0] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.b0, f.a0, acc[0][0], 0, 0, 2 * P, sb0, 2 * P, sa0);
-    acc[0][1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.b0, f.a1, acc[0][1], 0, 0, 2 * P, sb0, 2 * P, sa1);
-    acc[1][0] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.b1, f.a0, acc[1][0], 0, 0, 2 * P, sb1, 2 * P, sa0);
-    acc[1][1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.b1, f.a1, acc[1][1], 0, 0, 2 * P, sb1, 2 * P, sa1);
-    acc[2][0] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.b2, f.a0, acc[2][0], 0, 0, 2 * P, sb2, 2 * P, sa0);
-    acc[2][1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.b2, f.a1, acc[2][1], 0, 0, 2 * P, sb2, 2 * P, sa1);
-    acc[3][0] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.b3, f.a0, acc[3][0], 0, 0, 2 * P, sb3, 2 * P, sa0);
-    acc[3][1] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.b3, f.a1, acc[3][1], 0, 0, 2 * P, sb3, 2 * P, sa1);
+  auto read_frag = [&](int slot, Frags& f, int r) {
+    const uint8_t* st = lds + slot * S::kStageBytes;
+    const int k = r / (kMB + kNB), i = r % (kMB + kNB);
+    if (i < kMB) f.a[k][i] = frag(st + S::kOffA + k * S::kSliceA, (wm * kMB + i) * 32 + (lane & 31), c0, sw);
+    else f.b[k][i - kMB] = frag(st + S::kOffB + k * S::kSliceB, (wn * kNB + i - kMB) * 32 + (lane & 31), c0, sw);
+  };
+  auto mma = [&](const Frags& f, int x, auto pc) {  // product x of a stage; P: half of the 128-wide K tile (blocks 2P, 2P + 1)
+    const int k = x / (kMB * kNB), i = x / kMB % kNB, j = x % kMB;
+    const int sa = (int)(f.sa[j] >> sshift), sb = (int)(f.sb[i] >> sshift);
+    if ((S::kKS == 2 ? k : decltype(pc)::value) == 0)
+      acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.b[k][i], f.a[k][j], acc[i][j], 0, 0, 0, sb, 0, sa);
+    else
+      acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.b[k][i], f.a[k][j], acc[i][j], 0, 0, 2, sb, 2, sa);
   };
   // Steady state, branch-free (with conditional blocks the compiler sinks a stage's MFMAs below the next
   // barrier).  Step s: wait until stage s + 1 has landed (this wave's DMA) and this wave's reads of stage s are
@@ -371,33 +407,61 @@ __global__ __launch_bounds__(Shape<kNW>::kThreads) __attribute__((amdgpu_waves_p
     // Bare s_barrier: __syncthreads() adds a workgroup fence that waits for every outstanding DMA
     // (vmcnt(0)), which would drain the ring.
     __builtin_amdgcn_s_barrier();
-    issue_to(min(s + S::kStages, last), slot);
+    const int sn = min(s + S::kStages, last), dslot = slot;
     slot = slot + 1 == S::kStages ? 0 : slot + 1;
-    read(slot, nxt);
-    mma(cur, pc);
-    __builtin_amdgcn_sched_barrier(0);
+    read_scales(slot, nxt);
+    if constexpr (kMfma >= 8) {
+      // reads and DMAs spread evenly over all but the last MFMA, pinned in this order.  Starting the DMAs one MFMA
+      // late is 1% better for Tall and 1% worse for Wide; reads over 5 or 8 of the 8 MFMAs, DMAs over 4 or 5, DMAs
+      // only after half of them and s_setprio around each MFMA measured 0.5-6% slower.
+      constexpr int kOver = kMfma - 1, kD0 = S::kWaves == 8 ? 0 : 1;
+#pragma unroll
+      for (int x = 0; x < kMfma; ++x) {
+#pragma unroll
+        for (int r = kReads * x / kOver; r < kReads * (x + 1) / kOver && r < kReads; ++r) read_frag(slot, nxt, r);
+        if (x >= kD0) {
+#pragma unroll
+          for (int d = S::kDma * (x - kD0) / kOver; d < S::kDma * (x - kD0 + 1) / kOver && d < S::kDma; ++d)
+            dma(sn, dslot, d);
+        }
+        mma(cur, x, pc);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    } else {
+      issue_to(sn, dslot);
+#pragma unroll
+      for (int r = 0; r < kReads; ++r) read_frag(slot, nxt, r);
+#pragma unroll
+      for (int x = 0; x < kMfma; ++x) mma(cur, x, pc);
+      __builtin_amdgcn_sched_barrier(0);
+    }
   };
 
 #pragma unroll
-  for (int q = 0; q < S::kStages; ++q) issue_to(min(s_begin + q, last), q);
-  wait_vmcnt<(S::kStages - 1) * S::kDma>();  // stage s_begin landed
+  for (int q = 0; q < S::kStages; ++q) issue_to(min(s0 + q, last), q);
+  wait_vmcnt<(S::kStages - 1) * S::kDma>();  // stage s0 landed
   __builtin_amdgcn_s_barrier();
   Frags f0, f1;
-  read(0, f0);
-  for (int s = s_begin; s < s_end; s += 2) {
+  read_scales(0, f0);
+#pragma unroll
+  for (int r = 0; r < kReads; ++r) read_frag(0, f0, r);
+  int s = s0;
+  for (; s < last; s += 2) {
     step(s, f0, f1, std::integral_constant<int, 0>{});
     step(s + 1, f1, f0, std::integral_constant<int, 1>{});
   }
+  if constexpr (S::kKS == 2)  // an odd count of 128-wide K tiles
+    if (s == last) step(s, f0, f1, std::integral_constant<int, 0>{});
   wait_vmcnt<0>();  // drain the redundant tail loads before the workgroup can exit
 
-  if (part >= 0) {
+  if constexpr (std::is_same_v<S, Wide>) if (part >= 0) {
     // split tile: publish this piece, and let the last piece to arrive finish the tile
     const int st_ = tile - plan.full;
     float4* wsp = plan.ws + (((int64_t)st_ * plan.parts + part) * S::kWaves + wave) * (32 * 64) + lane;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < kNB; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < kMB; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q)
           wsp[((i * 2 + j) * 4 + q) * 64] =
@@ -410,9 +474,9 @@ __global__ __launch_bounds__(Shape<kNW>::kThreads) __attribute__((amdgpu_waves_p
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");  // see the other pieces' stores
     const float4* wsb = plan.ws + ((int64_t)st_ * plan.parts * S::kWaves + wave) * (32 * 64) + lane;
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+    for (int i = 0; i < kNB; ++i)
 #pragma unroll
-      for (int j = 0; j < 2; ++j)
+      for (int j = 0; j < kMB; ++j)
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
           float4 t = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -440,12 +504,14 @@ __global__ __launch_bounds__(Shape<kNW>::kThreads) __attribute__((amdgpu_waves_p
     // now), so the epilogue waits for one memory latency instead of one per product.
     constexpr int R = kR, H = R / 16;
     const int Nf = swe.N, lg = lane >> 5, rho = lane & 31;
-    const int t64 = n0 >> 1;                      // first gate / up column of the tile: 64 * (n0 / 128)
+    static_assert(kNB == 4, "a wave holds gate and up of the same columns");
+    const int nw = n0 + wn * 128;                 // the wave's 128 output columns
+    const int t64 = nw >> 1;                      // their first gate / up column: 64 * (nw / 128)
     const int srows = (M + 127) / 128 * 128;      // rows of the blocked scale buffer of h
-    v8bf xg[2][H], xu[2][H], wg[2][H], wu[2][H], af[2][2];
+    v8bf xg[kMB][H], xu[kMB][H], wg[2][H], wu[2][H], af[2][2];
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-      const int mc = min(m0 + wm * 64 + mt * 32 + (lane & 31), M - 1);
+    for (int mt = 0; mt < kMB; ++mt) {
+      const int mc = min(m0 + (wm * kMB + mt) * 32 + (lane & 31), M - 1);
 #pragma unroll
       for (int h = 0; h < H; ++h) {
         xg[mt][h] = load_bf8(swe.xs + (int64_t)mc * 2 * R + h * 16 + lg * 8);
@@ -468,8 +534,8 @@ __global__ __launch_bounds__(Shape<kNW>::kThreads) __attribute__((amdgpu_waves_p
       }
     }
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-      const int m = m0 + wm * 64 + mt * 32 + (lane & 31);
+    for (int mt = 0; mt < kMB; ++mt) {
+      const int m = m0 + (wm * kMB + mt) * 32 + (lane & 31);
       const bool live = m < M;
       v16f xacc = v16f{};  // xS_down partial D[ρ][m] over the tile's 64 columns
 #pragma unroll
@@ -527,7 +593,7 @@ __global__ __launch_bounds__(Shape<kNW>::kThreads) __attribute__((amdgpu_waves_p
               af[b][ks], as_bf8(make_uint4(hw[4 * ks], hw[4 * ks + 1], hw[4 * ks + 2], hw[4 * ks + 3])), xacc, 0, 0, 0);
       }
       if (live) {  // lane l holds ρ = g*8 + (l/32)*4 + 0..3 in registers 4g..4g+3: one 16-byte store per g < R/8
-        float* pp = swe.part + ((int64_t)(n0 >> 7) * M + m) * R + lg * 4;
+        float* pp = swe.part + ((int64_t)(nw >> 7) * M + m) * R + lg * 4;
 #pragma unroll
         for (int g4 = 0; g4 < R / 8; ++g4)
           *reinterpret_cast<float4*>(pp + g4 * 8) =
@@ -552,6 +618,7 @@ __global__ __launch_bounds__(Shape<kNW>::kThreads) __attribute__((amdgpu_waves_p
     // (the memory counter completes in order); the small per-row operands are loaded once per row block and the
     // weights are staged in LDS once per tile.
     constexpr int R = kR;
+    static_assert(std::is_same_v<S, Tall>, "256-row partials of 128-column tiles");
     static_assert(R == 16, "the backward epilogue's LDS is laid out for r = 16");
     const int lg = lane >> 5, rho = lane & 31;
     const int Tpad = (M + 127) / 128 * 128;  // rows of the transposed operands and of the scale buffer
@@ -785,31 +852,31 @@ __global__ __launch_bounds__(Shape<kNW>::kThreads) __attribute__((amdgpu_waves_p
   const int ncol0 = cseg.col0[sg];
   const uint16_t* const lp = lora.p + cseg.rcol[sg];  // the segment's rank-r columns of P and Q
   const uint16_t* const lq = lora.q + cseg.rcol[sg];
-  // epilogue: lane holds row m = m0 + wm*64 + mt*32 + lane%32 and columns n0 + wn*128 + nt*32 + g*8 +
+  // epilogue: lane holds row m = m0 + (wm*kMB + mt)*32 + lane%32 and columns n0 + (wn*kNB + nt)*32 + g*8 +
   // (lane/32)*4 + 0..3 in acc[nt][mt][4g .. 4g+3]; with B in the pi_col order (b_pi) the 16 contiguous columns
-  // n0 + wn*128 + nt*32 + (lane/32)*16 + i in acc[nt][mt][i].
+  // n0 + (wn*kNB + nt)*32 + (lane/32)*16 + i in acc[nt][mt][i].
   // The rank-r operands: the P rows of both row halves are loaded first, the Q rows of column block nt + 1 while
   // block nt is finished, so the wave waits for one memory latency, not one per 32 x 32 block.  Rounding to bf16
   // goes through v_cvt_pk_bf16_f32 (rnd2), pairwise.
   constexpr int kH = kR > 0 ? kR / 16 : 1;
-  v8bf pf[2][kH], qf[2][kH];
+  v8bf pf[kMB][kH], qf[2][kH];
   auto load_q = [&](int nt, v8bf* dst) {
-    const int nr = min(n0 + wn * 128 + nt * 32 + (b_pi ? pi_col(lane & 31) : (lane & 31)), N - 1);
+    const int nr = min(n0 + (wn * kNB + nt) * 32 + (b_pi ? pi_col(lane & 31) : (lane & 31)), N - 1);
 #pragma unroll
     for (int h = 0; h < kH; ++h)
       dst[h] = *reinterpret_cast<const v8bf*>(lq + (int64_t)nr * lora.ld_q + h * 16 + (lane >> 5) * 8);
   };
   if constexpr (kR > 0) {
     bool p_ready = true;  // P summed in this launch: its rows published, or this tile sums them (presum_device.h)
-    if constexpr (kFoldSum<kR, kNW, kEpi>) {
+    if constexpr (kFoldSum<kR, S, kEpi>) {
       if (pre.blocks) p_ready = presum_wait(pre, m0, min(m0 + kBM, M), &arrived);
     }
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-      const int mc = min(m0 + wm * 64 + mt * 32 + (lane & 31), M - 1);
+    for (int mt = 0; mt < kMB; ++mt) {
+      const int mc = min(m0 + (wm * kMB + mt) * 32 + (lane & 31), M - 1);
 #pragma unroll
       for (int h = 0; h < kH; ++h) {
-        if constexpr (kFoldSum<kR, kNW, kEpi>) {
+        if constexpr (kFoldSum<kR, S, kEpi>) {
           if (pre.blocks) {
             pf[mt][h] = p_ready ? presum_load8(lp + (int64_t)mc * lora.ld_p + h * 16 + (lane >> 5) * 8)
                                 : presum_row8(pre, mc, h * 16 + (lane >> 5) * 8, kR);
@@ -822,14 +889,14 @@ __global__ __launch_bounds__(Shape<kNW>::kThreads) __attribute__((amdgpu_waves_p
     load_q(0, qf[0]);
   }
 #pragma unroll
-  for (int nt = 0; nt < 4; ++nt) {
-    const int nb = n0 + wn * 128 + nt * 32;
+  for (int nt = 0; nt < kNB; ++nt) {
+    const int nb = n0 + (wn * kNB + nt) * 32;
     if constexpr (kR > 0) {
-      if (nt + 1 < 4) load_q(nt + 1, qf[(nt + 1) & 1]);
+      if (nt + 1 < kNB) load_q(nt + 1, qf[(nt + 1) & 1]);
     }
 #pragma unroll
-    for (int mt = 0; mt < 2; ++mt) {
-      const int m = m0 + wm * 64 + mt * 32 + (lane & 31);
+    for (int mt = 0; mt < kMB; ++mt) {
+      const int m = m0 + (wm * kMB + mt) * 32 + (lane & 31);
       const v16f o = acc[nt][mt];
       uint32_t wv[8];  // packed bf16 pairs of o[2k], o[2k + 1]
       if constexpr (kR > 0) {
@@ -888,14 +955,13 @@ int cached_cus() {
   return cus[dev];
 }
 
-// Split the tail wave along K when it would leave more than half of the workgroup slots idle (slots = CUs x
-// workgroups per CU: the LDS ring takes 136 KB at kNW = 2, 78 KB at kNW = 1).  Returns the workspace bytes
-// the plan needs (0 without a split).
-template <int kNW>
+// Split the tail wave of the Wide shape along K when it would leave more than half of the CUs idle (one workgroup
+// per CU).  Returns the workspace bytes the plan needs (0 without a split).
+template <class S>
 int64_t make_plan(int64_t M, int64_t N, int64_t K, int cus, Plan& p) {
-  using S = Shape<kNW>;
-  const int slots = cus * (kNW == 2 ? 1 : 2);
-  p.tm = (int)((M + kBM - 1) / kBM);
+  constexpr bool kSplit = std::is_same_v<S, Wide>;
+  const int slots = cus;
+  p.tm = (int)((M + S::kBM - 1) / S::kBM);
   p.tn = (int)((N + S::kBN - 1) / S::kBN);
   const int total = p.tm * p.tn, ns = (int)(K / kBK);
   const int rem = total % slots;
@@ -905,7 +971,7 @@ int64_t make_plan(int64_t M, int64_t N, int64_t K, int cus, Plan& p) {
   p.chunk = ns;
   // Two co-resident workgroups per CU already overlap one tile's pipeline fill and epilogue with the other's
   // main loop; splitting the tail along K measured slower there (down: 184-199 us split vs 143-149 whole).
-  if (kNW == 2 && rem > 0 && 2 * rem <= slots && rem <= kMaxSplitTiles) {
+  if (kSplit && rem > 0 && 2 * rem <= slots && rem <= kMaxSplitTiles) {
     int parts = min(kMaxParts, slots / rem);
     int chunk = 2 * ((ns + 2 * parts - 1) / (2 * parts));
     parts = (ns + chunk - 1) / chunk;
@@ -922,18 +988,17 @@ int64_t make_plan(int64_t M, int64_t N, int64_t K, int cus, Plan& p) {
   return kCounterBytes + (int64_t)p.nsplit * p.parts * S::kPartBytes;
 }
 
-template <int kNW>
+template <class S>
 void launch(const uint8_t* A, const uint8_t* SA, int64_t lda, const uint8_t* B, const uint8_t* SB, int64_t ldb,
             int M, int N, int K, const CSeg& cseg, const Lora& lo, int r, const Plan& plan, int layout,
             const TnBatch& tnb, int64_t tn_blocks, const PreSum& pre, hipStream_t stm) {
-  using S = Shape<kNW>;
   dim3 grid((unsigned)(pre.blocks + 8 * plan.per_full + 8 * plan.per_split + tn_blocks));
 #define GEMM_ARGS A, SA, lda, B, SB, ldb, M, N, K, cseg, lo, plan, layout, SwEpi{}, SwBwd{}, tnb, pre
-  if (!lo.p) gemm_kernel<0, kNW, kEpiPlain><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
-  else if (r == 16) gemm_kernel<16, kNW, kEpiPlain><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
-  else if (r == 32) gemm_kernel<32, kNW, kEpiPlain><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
-  else if (r == 48) gemm_kernel<48, kNW, kEpiPlain><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
-  else gemm_kernel<64, kNW, kEpiPlain><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
+  if (!lo.p) gemm_kernel<0, S, kEpiPlain><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
+  else if (r == 16) gemm_kernel<16, S, kEpiPlain><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
+  else if (r == 32) gemm_kernel<32, S, kEpiPlain><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
+  else if (r == 48) gemm_kernel<48, S, kEpiPlain><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
+  else gemm_kernel<64, S, kEpiPlain><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
 #undef GEMM_ARGS
 }
 
@@ -942,7 +1007,7 @@ void launch(const uint8_t* A, const uint8_t* SA, int64_t lda, const uint8_t* B, 
 extern "C" int64_t mxfp8_gemm_workspace_size(int64_t M, int64_t N, int64_t K) {
   if (M <= 0 || N <= 0 || K <= 0 || K % 128 || N % 128) return 0;
   Plan p;
-  return make_plan<2>(M, N, K, cached_cus(), p);  // only the 8-wave shape splits
+  return make_plan<Wide>(M, N, K, cached_cus(), p);  // only the 8-wave shape splits
 }
 
 namespace {
@@ -985,8 +1050,9 @@ int gemm_impl(const void* a, const void* sa, int64_t lda, const void* b, const v
   }
   if (M == 0) return MXFP8_OK;
   Plan plan;
+  const int cus = cached_cus();
   const bool wide = layout & MXFP8_GEMM_WIDE;
-  const int64_t need = wide ? make_plan<2>(M, N, K, cached_cus(), plan) : make_plan<1>(M, N, K, cached_cus(), plan);
+  const int64_t need = wide ? make_plan<Wide>(M, N, K, cus, plan) : make_plan<Tall>(M, N, K, cus, plan);
   if (need > workspace_bytes) {  // no (or too small a) workspace: run every tile whole
     plan.full = plan.tm * plan.tn;
     plan.per_full = (plan.full + 7) / 8;
@@ -999,12 +1065,12 @@ int gemm_impl(const void* a, const void* sa, int64_t lda, const void* b, const v
   Lora lo{(const uint16_t*)lora_p, ld_p, (const uint16_t*)lora_q, ld_q, alpha};
   const uint8_t *A = (const uint8_t*)a, *SA = (const uint8_t*)sa, *B = (const uint8_t*)b, *SB = (const uint8_t*)sb;
   const int tiled = (int)(layout & ~MXFP8_GEMM_WIDE);
-  if (wide)
-    launch<2>(A, SA, lda, B, SB, ldb, (int)M, (int)N, (int)K, cseg, lo, (int)r, plan, tiled, tnb, 0, PreSum{},
-              (hipStream_t)stream);
-  else
-    launch<1>(A, SA, lda, B, SB, ldb, (int)M, (int)N, (int)K, cseg, lo, (int)r, plan, tiled, tnb, tn_blocks, pre,
-              (hipStream_t)stream);
+  hipStream_t stm = (hipStream_t)stream;
+#define GEMM_LAUNCH(S) \
+  launch<S>(A, SA, lda, B, SB, ldb, (int)M, (int)N, (int)K, cseg, lo, (int)r, plan, tiled, tnb, tn_blocks, pre, stm)
+  if (wide) GEMM_LAUNCH(Wide);
+  else GEMM_LAUNCH(Tall);
+#undef GEMM_LAUNCH
   MX_CHECK_LAUNCH("mxfp8_gemm_nt");
   return MXFP8_OK;
 }
@@ -1037,7 +1103,7 @@ extern "C" int mxfp8_gemm_nt_tn(const void* a, const void* sa, int64_t lda, cons
   int64_t nb = 0, ns = 0;
   int rc = tn_batch_tables("mxfp8_gemm_nt_tn", jobs, n_jobs, T_tn, K_tn, chunks, part, tnb, sa_tn, nb, ns);
   if (rc != MXFP8_OK) return rc;
-  MX_CHECK_ARG(nb + (M + kBM - 1) / kBM * (N / 128) + 8 < (1LL << 31), "mxfp8_gemm_nt_tn: too many workgroups");
+  MX_CHECK_ARG(nb + (M + 255) / 256 * (N / 128) + 8 < (1LL << 31), "mxfp8_gemm_nt_tn: too many workgroups");
   CSeg cs{};
   cs.n = 1;
   cs.ptr[0] = (uint16_t*)c;
@@ -1180,7 +1246,7 @@ extern "C" int mxfp8_gemm_swiglu_fwd(const void* a, const void* sa, const void* 
                    mx_aligned(gu, 16) && mx_aligned(q_h, 16) && mx_aligned(part, 16),
                "mxfp8_gemm_swiglu_fwd: misaligned buffer");
   Plan plan;
-  make_plan<1>(M, 2 * N, K, cached_cus(), plan);
+  make_plan<Tall>(M, 2 * N, K, cached_cus(), plan);
   SwEpi sw{(const uint16_t*)xs, (const uint16_t*)bg, (const uint16_t*)bu, (const uint16_t*)ad, s_g, s_u,
            (uint16_t*)gu, (uint8_t*)q_h, (uint8_t*)s_h, part, (int)N};
   CSeg cs{};
@@ -1189,12 +1255,12 @@ extern "C" int mxfp8_gemm_swiglu_fwd(const void* a, const void* sa, const void* 
   const int tiled = MXFP8_GEMM_A_TILED | MXFP8_GEMM_B_TILED;
   hipStream_t stm = (hipStream_t)stream;
   const uint8_t *A = (const uint8_t*)a, *SA = (const uint8_t*)sa, *B = (const uint8_t*)b, *SB = (const uint8_t*)sb;
-  if (r == 16)
-    gemm_kernel<16, 1, kEpiSwiGluFwd><<<grid, Shape<1>::kThreads, 0, stm>>>(
-        A, SA, K, B, SB, K, (int)M, (int)(2 * N), (int)K, cs, Lora{}, plan, tiled, sw, SwBwd{}, TnBatch{}, PreSum{});
-  else
-    gemm_kernel<32, 1, kEpiSwiGluFwd><<<grid, Shape<1>::kThreads, 0, stm>>>(
-        A, SA, K, B, SB, K, (int)M, (int)(2 * N), (int)K, cs, Lora{}, plan, tiled, sw, SwBwd{}, TnBatch{}, PreSum{});
+#define SWIGLU_LAUNCH(R, S)                                                                                        \
+  gemm_kernel<R, S, kEpiSwiGluFwd><<<grid, S::kThreads, 0, stm>>>(A, SA, K, B, SB, K, (int)M, (int)(2 * N), (int)K, cs, \
+                                                                  Lora{}, plan, tiled, sw, SwBwd{}, TnBatch{}, PreSum{})
+  if (r == 16) SWIGLU_LAUNCH(16, Tall);
+  else SWIGLU_LAUNCH(32, Tall);
+#undef SWIGLU_LAUNCH
   MX_CHECK_LAUNCH("mxfp8_gemm_swiglu_fwd");
   return MXFP8_OK;
 }
@@ -1221,7 +1287,7 @@ extern "C" int mxfp8_gemm_swiglu_bwd(const void* a, const void* sa, const void* 
                    mx_aligned(dad_part, 16),
                "mxfp8_gemm_swiglu_bwd: misaligned buffer");
   Plan plan;
-  make_plan<1>(M, N, K, cached_cus(), plan);
+  make_plan<Tall>(M, N, K, cached_cus(), plan);
   SwBwd sw{(const uint16_t*)gu,  (const uint16_t*)xs,  (const uint16_t*)xsT, (const uint16_t*)dxd,
            (const uint16_t*)dxdT, (const uint16_t*)bg, (const uint16_t*)bgT, (const uint16_t*)bu,
            (const uint16_t*)buT, (const uint16_t*)ad,  (const uint16_t*)adT, s_g, s_u, (uint8_t*)q, (uint8_t*)s,
@@ -1230,7 +1296,7 @@ extern "C" int mxfp8_gemm_swiglu_bwd(const void* a, const void* sa, const void* 
   cs.n = 1;
   const dim3 grid((unsigned)(8 * plan.per_full));
   const int tiled = MXFP8_GEMM_A_TILED | MXFP8_GEMM_B_TILED;
-  gemm_kernel<16, 1, kEpiSwiGluBwd><<<grid, Shape<1>::kThreads, 0, (hipStream_t)stream>>>(
+  gemm_kernel<16, Tall, kEpiSwiGluBwd><<<grid, Tall::kThreads, 0, (hipStream_t)stream>>>(
       (const uint8_t*)a, (const uint8_t*)sa, K, (const uint8_t*)b, (const uint8_t*)sb, K, (int)M, (int)N, (int)K, cs,
       Lora{}, plan, tiled, SwEpi{}, sw, TnBatch{}, PreSum{});
   MX_CHECK_LAUNCH("mxfp8_gemm_swiglu_bwd");
