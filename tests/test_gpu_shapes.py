@@ -1,0 +1,72 @@
+"""The workgroup shapes of the MX GEMM (csrc/mx_gemm.hip, pick_shape): 64 x 64, 64 x 128 and 128 x 128 tiles where
+256 x 128 ones would leave CUs idle, 256 x 256 for long launches.  An output element adds the same products over K in
+the same order in every shape, so each size must give the bits of the explicitly asked 8-wave shape run whole
+(MXFP8_GEMM_WIDE without a workspace), which every size takes: bit-exact, no tolerance."""
+import pytest
+import torch
+
+import _native
+import mxfp8
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(M, N, K, gpu):
+    g = torch.Generator(device=gpu).manual_seed(M + 3 * N + 7 * K)
+    e = torch.exp2(torch.randint(-6, 6, (M, 1), device=gpu, generator=g).float())
+    a = (torch.randn(M, K, device=gpu, generator=g) * e).to(torch.bfloat16)
+    b = (torch.randn(N, K, device=gpu, generator=g) * 0.02).to(torch.bfloat16)
+    return g, mxfp8.mx_quant_tiled(a), mxfp8.mx_quant_tiled(b), b
+
+
+# edges of 64, 128 and 256 rows; N that is and is not a multiple of 256; an odd count of 128-wide K tiles
+@pytest.mark.parametrize("M,N,K", [
+    (1, 128, 128), (63, 256, 384), (64, 1024, 1024), (65, 384, 640), (129, 2048, 1152),    # 64 x 64
+    (1000, 2048, 1024), (961, 1920, 1408),                                                 # 64 x 128
+    (129, 12288, 256), (1500, 2048, 2048), (1921, 1920, 1152),                             # 128 x 128
+    (321, 12288, 384), (1025, 12288, 128),                                                 # 256 x 128
+    (5000, 2048, 2048), (4353, 2304, 1280)])                                               # 256 x 256
+@pytest.mark.parametrize("rank", [0, 16, 48])
+def test_every_shape_gives_the_same_bits(M, N, K, rank, gpu):
+    g, (qa, sa), (qb, sb), b = _operands(M, N, K, gpu)
+    lora = None
+    if rank:
+        lora = ((torch.randn(M, rank, device=gpu, generator=g) * 0.1).to(torch.bfloat16),
+                (torch.randn(N, rank, device=gpu, generator=g) * 0.1).to(torch.bfloat16))
+    want = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=gpu)
+    _native.gemm_nt(qa, sa, K, qb, sb, K, M, N, K, want, lora=lora, alpha=0.7, split=False, layout=3 | _native.GEMM_WIDE)
+    got = mxfp8.mx_mm(qa, sa, qb, sb, lora=lora, alpha=0.7, layout=3, m=M)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    # the pi_col row order of B (16-byte stores)
+    qp, sp = mxfp8.mx_quant_tiled(b[mxfp8.fused_dgrad_rows(N, gpu)].contiguous())
+    got = mxfp8.mx_mm(qa, sa, qp, sp, lora=lora, alpha=0.7, layout=3 | _native.GEMM_B_PI, m=M)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    # C in the fused-tile layout (rows past M are not written: both start from zeros)
+    ft = [torch.zeros((mxfp8.ft_rows(M), N), dtype=torch.bfloat16, device=gpu) for _ in range(2)]
+    _native.gemm_nt(qa, sa, K, qb, sb, K, M, N, K, ft[0], lora=lora, alpha=0.7, split=False,
+                    layout=3 | _native.GEMM_WIDE | _native.GEMM_C_FT)
+    mxfp8.mx_mm(qa, sa, qp, sp, out=ft[1], lora=lora, alpha=0.7, layout=3 | _native.GEMM_B_PI | _native.GEMM_C_FT, m=M)
+    assert torch.equal(ft[0].view(torch.int16), ft[1].view(torch.int16))
+
+
+@pytest.mark.parametrize("M,N,K", [(65, 384, 640), (961, 1920, 1408), (1921, 1920, 1152), (20501, 2048, 12288)])
+def test_folded_launches_in_every_shape(M, N, K, gpu):
+    """mxfp8_gemm_nt_sum and mxfp8_gemm_nt_tn against the separate calls, in the shapes that carry the folded work and
+    in the 8-wave one, which launches it apart: bit-identical."""
+    g, (qa, sa), (qb, sb), _ = _operands(M, N, K, gpu)
+    part = torch.randn(5, M, 16, device=gpu, generator=g)
+    Q = (torch.randn(N, 32, device=gpu, generator=g) * 0.1).to(torch.bfloat16)
+    P = torch.empty(M, 16, dtype=torch.bfloat16, device=gpu)
+    _native.sum_parts(part, 5, M * 16, P)
+    want = mxfp8.mx_mm(qa, sa, qb, sb, lora=(P, Q[:, :16]), alpha=0.5, layout=3, m=M)
+    P2 = torch.empty_like(P)
+    got = mxfp8.mx_mm_sum(qa, sa, qb, sb, part, P2, Q[:, :16], 0.5, 3, M)
+    assert torch.equal(P, P2) and torch.equal(got.view(torch.int16), want.view(torch.int16))
+    x = torch.randn(M, 256, device=gpu, generator=g).to(torch.bfloat16)
+    P3 = torch.randn(M, 32, device=gpu, generator=g).to(torch.bfloat16)
+    outs = [torch.empty(32, 256, dtype=torch.bfloat16, device=gpu) for _ in range(2)]
+    scratch = torch.empty(_native.lora_tn_chunks(M, 256) * 32 * 256, dtype=torch.float32, device=gpu)
+    want = mxfp8.mx_mm(qa, sa, qb, sb, lora=(P3, Q), alpha=1.0, layout=3, m=M)
+    _native.lora_tn_batch([(x, P3, outs[0], 1.0, False)], scratch)
+    got = mxfp8.mx_mm_tn(qa, sa, qb, sb, (P3, Q), 1.0, 3, M, [(x, P3, outs[1], 1.0, False)], scratch)
+    assert torch.equal(outs[0], outs[1]) and torch.equal(got.view(torch.int16), want.view(torch.int16))

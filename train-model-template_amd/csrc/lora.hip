@@ -1067,20 +1067,25 @@ int tn_sum_batch_launch(const TnSumBatch& sa, int64_t ns, hipStream_t stm, const
 
 }  // namespace mxk
 
+int mxk::tn_batch_launch(const TnBatch& a, int64_t nb, hipStream_t stm, const char* who) {
+  if (a.kd == 2 && a.wide) tn_batch_kernel<2, true><<<(unsigned)nb, 256, 0, stm>>>(a);
+  else if (a.kd == 2) tn_batch_kernel<2, false><<<(unsigned)nb, 256, 0, stm>>>(a);
+  else if (a.wide) tn_batch_kernel<1, true><<<(unsigned)nb, 256, 0, stm>>>(a);
+  else tn_batch_kernel<1, false><<<(unsigned)nb, 256, 0, stm>>>(a);
+  MX_CHECK_LAUNCH(who);
+  return MXFP8_OK;
+}
+
 extern "C" int mxfp8_lora_tn_batch(const mxfp8_lora_tn_job* jobs, int64_t n_jobs, int64_t T, int64_t K,
                                    int64_t chunks, float* part, void* stream) {
   TnBatch a;
   TnSumBatch sa;
   int64_t nb = 0, ns = 0;
-  const int rc = tn_batch_tables("mxfp8_lora_tn_batch", jobs, n_jobs, T, K, chunks, part, a, sa, nb, ns);
+  int rc = tn_batch_tables("mxfp8_lora_tn_batch", jobs, n_jobs, T, K, chunks, part, a, sa, nb, ns);
   if (rc != MXFP8_OK) return rc;
-  hipStream_t stm = (hipStream_t)stream;
-  if (a.kd == 2 && a.wide) tn_batch_kernel<2, true><<<(unsigned)nb, 256, 0, stm>>>(a);
-  else if (a.kd == 2) tn_batch_kernel<2, false><<<(unsigned)nb, 256, 0, stm>>>(a);
-  else if (a.wide) tn_batch_kernel<1, true><<<(unsigned)nb, 256, 0, stm>>>(a);
-  else tn_batch_kernel<1, false><<<(unsigned)nb, 256, 0, stm>>>(a);
-  MX_CHECK_LAUNCH("mxfp8_lora_tn_batch");
-  return tn_sum_batch_launch(sa, ns, stm, "mxfp8_lora_tn_batch");
+  rc = mxk::tn_batch_launch(a, nb, (hipStream_t)stream, "mxfp8_lora_tn_batch");
+  if (rc != MXFP8_OK) return rc;
+  return tn_sum_batch_launch(sa, ns, (hipStream_t)stream, "mxfp8_lora_tn_batch");
 }
 
 // ------------------------------------------------------------------ allocation-free token reduction

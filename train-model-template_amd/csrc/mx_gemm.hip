@@ -20,6 +20,12 @@
 // workgroup per CU (T = 256, K = 12288) 66 -> 57; Wide at T = 142336: dx 2692 -> 2568, down 1406 -> 1366.  All
 // outputs are bit-identical.
 //
+// Sizes that leave CUs idle take smaller tiles (Mid, Low, Small): a lone workgroup's step costs its serial part
+// (barrier, fragment reads, their wait: about 0.13 us, whatever the ring's depth) besides its MFMAs, so a launch of
+// few tiles takes (K steps) x (0.30, 0.23, 0.15, 0.12 us) at 256 x 128, 128 x 128, 64 x 128, 64 x 64, and Low and
+// Small take 128-wide K steps, half the barriers.  Long launches take Wide, which reads a third less per flop from
+// L2.  pick_shape chooses.
+//
 // What bounds it (rocprofv3 counters on the MLP GEMMs): the CU's vector-memory path that carries the
 // operand DMA (TA / TD busy 65-89% of the kernel, TD waiting on L1/L2 data about 45% of the time) while the
 // matrix pipe is busy ~48%.  LDS reads overlap MFMAs well on gfx950 (a software-pipelined fragment-read +
@@ -102,6 +108,9 @@ struct Shape {
 };
 using Tall = Shape<2, 4, 4, 1, 1, 3>;   // 256 x 128, 4 waves, ring 78 KB: two workgroups per CU
 using Wide = Shape<2, 4, 4, 2, 1, 4>;   // 256 x 256, 8 waves, ring 136 KB: one workgroup per CU
+using Mid = Shape<1, 4, 4, 1, 1, 3>;    // 128 x 128, 4 waves, ring 51 KB: three per CU
+using Low = Shape<1, 2, 2, 2, 2, 3>;    // 64 x 128, 4 waves, ring 75 KB: two per CU
+using Small = Shape<1, 1, 2, 2, 2, 4>;  // 64 x 64, 4 waves, ring 68 KB: two per CU
 
 struct Lora {
   const uint16_t* p;  // [M, r] bf16
@@ -212,7 +221,8 @@ template <int kR, class S, int kEpi>
 constexpr bool kFoldSum = kR == 16 && S::kThreads == 256 && kEpi == 0;
 template <class S>
 constexpr bool kTnFits = tn_batch_lds_elems<true>() * 2 <= S::kStages * S::kStageBytes;
-static_assert(kTnFits<Tall>, "the folded token reduction borrows the 4-wave ring's LDS");
+static_assert(kTnFits<Tall> && kTnFits<Mid> && kTnFits<Low> && kTnFits<Small>,
+              "the folded token reduction borrows the 4-wave ring's LDS");
 
 // n scale words (4-byte aligned to their count) from LDS
 template <int n>
@@ -1002,6 +1012,54 @@ void launch(const uint8_t* A, const uint8_t* SA, int64_t lda, const uint8_t* B, 
 #undef GEMM_ARGS
 }
 
+enum class ShapeId { kTall, kWide, kMid, kLow, kSmall };
+
+// Estimated us of a launch in one shape, from the size alone: with w = tiles per CU and rounds = ceil(w),
+//   K steps * (step * rounds + fill * w + (one round: lone) + late * max(0, w - 8)) + round * rounds + base.
+// A round costs its K steps' serial part (barrier, fragment reads) whether or not it fills the chip (`step`), the
+// rest grows with the tiles (`fill`); `late` is what long launches lose to the L2 and the clock.  Least squares
+// over 13 shapes (N 1024-12288, K 1024-12288) at 20 values of M from 64 to 142336, on one MI355X: relative error
+// 3-4% (standard deviation); over those sizes the shape it picks takes 0.2% longer than the fastest one on average.
+struct ShapeCost {
+  int bm, bn;
+  float step, fill, lone, late, round, base;
+};
+constexpr ShapeCost kCost[] = {{256, 128, 0.2041f, 0.1618f, 0.0282f, 0.0512f, 2.99f, 2.15f},   // Tall
+                               {256, 256, 0.3247f, 0.3712f, 0.0002f, 0.0379f, 7.46f, 1.29f},   // Wide
+                               {128, 128, 0.1471f, 0.0780f, 0.0449f, 0.0f, 1.76f, 2.05f},      // Mid
+                               {64, 128, 0.1043f, 0.0421f, 0.0217f, 0.0f, 1.08f, 2.12f},       // Low
+                               {64, 64, 0.0770f, 0.0204f, 0.0190f, 0.0f, 0.70f, 2.23f}};       // Small
+
+float shape_us(ShapeId id, int64_t M, int64_t N, int64_t K, int cus) {
+  const ShapeCost& c = kCost[(int)id];
+  const int64_t tiles = ((M + c.bm - 1) / c.bm) * ((N + c.bn - 1) / c.bn);
+  const float w = (float)tiles / cus, rounds = (float)((tiles + cus - 1) / cus);
+  return (float)(K / kBK) * (c.step * rounds + c.fill * w + (rounds == 1.f ? c.lone : 0.f) + c.late * std::max(0.f, w - 8)) +
+         c.round * rounds + c.base;
+}
+
+// The shape of a plain GEMM (its bits are the same in every shape: an output element's products are added over K in
+// the same order).  us per launch, Tall / the shape taken: M = 256, N = 2048, K = 12288 57 / 23 (Small); M = 1000,
+// N = 2048, K = 6144 32 / 21 (Low); M = 2048, N = 2048, K = 6144 32.2 / 30.7 (Mid); M = 21504, N = 2048, K = 12288
+// 462 / 412 (Wide).  Another shape than Tall has to be 2% faster by the estimate.  wide_ok: N % 256 == 0 and one
+// output; wide_more: us that the launches which Wide cannot fold into its own cost.
+ShapeId pick_shape(int64_t M, int64_t N, int64_t K, int cus, bool wide_ok, float wide_more) {
+  ShapeId best = ShapeId::kTall;
+  float t = shape_us(best, M, N, K, cus) * 0.98f;
+  for (ShapeId id : {ShapeId::kWide, ShapeId::kMid, ShapeId::kLow, ShapeId::kSmall}) {
+    if (id == ShapeId::kWide && !(wide_ok && N % 256 == 0)) continue;
+    const float e = shape_us(id, M, N, K, cus) + (id == ShapeId::kWide ? wide_more : 0.f);
+    if (e < t) {
+      best = id;
+      t = e;
+    }
+  }
+  return best;
+}
+// us of a token reduction or a partial sum in a launch of its own beyond its share of a folded launch (measured at
+// T = 10752: dx with its reductions 252 folded, 237 + 29 apart; down with its sum 135 against 124 + 13).
+constexpr float kUnfoldedTn = 12.f, kUnfoldedSum = 2.f;
+
 }  // namespace
 
 extern "C" int64_t mxfp8_gemm_workspace_size(int64_t M, int64_t N, int64_t K) {
@@ -1015,7 +1073,7 @@ namespace {
 int gemm_impl(const void* a, const void* sa, int64_t lda, const void* b, const void* sb, int64_t ldb, int64_t M,
               int64_t N, int64_t K, CSeg cseg, const void* lora_p, int64_t ld_p, const void* lora_q, int64_t ld_q,
               int64_t r, float alpha, int64_t layout, void* workspace, int64_t workspace_bytes, void* stream,
-              const TnBatch& tnb = TnBatch{}, int64_t tn_blocks = 0, const PreSum& pre = PreSum{}) {
+              const TnBatch& tnb = TnBatch{}, int64_t tn_blocks = 0, const PreSum& pre = PreSum{}, int shape_id = -1) {
   void* const c = cseg.ptr[0];
   int64_t ldc = cseg.ld[0];
   MX_CHECK_ARG(a && sa && b && sb && c, "mxfp8_gemm_nt: null pointer");
@@ -1052,8 +1110,18 @@ int gemm_impl(const void* a, const void* sa, int64_t lda, const void* b, const v
   Plan plan;
   const int cus = cached_cus();
   const bool wide = layout & MXFP8_GEMM_WIDE;
-  const int64_t need = wide ? make_plan<Wide>(M, N, K, cus, plan) : make_plan<Tall>(M, N, K, cus, plan);
-  if (need > workspace_bytes) {  // no (or too small a) workspace: run every tile whole
+  const ShapeId shape = wide            ? ShapeId::kWide
+                        : shape_id >= 0 ? (ShapeId)shape_id
+                                        : pick_shape(M, N, K, cus, cseg.n == 1, 0.f);
+  int64_t need = 0;
+  switch (shape) {
+    case ShapeId::kTall: need = make_plan<Tall>(M, N, K, cus, plan); break;
+    case ShapeId::kWide: need = make_plan<Wide>(M, N, K, cus, plan); break;
+    case ShapeId::kMid: need = make_plan<Mid>(M, N, K, cus, plan); break;
+    case ShapeId::kLow: need = make_plan<Low>(M, N, K, cus, plan); break;
+    case ShapeId::kSmall: need = make_plan<Small>(M, N, K, cus, plan); break;
+  }
+  if (need > workspace_bytes || (need && !wide)) {  // no (or too small a) workspace: run every tile whole
     plan.full = plan.tm * plan.tn;
     plan.per_full = (plan.full + 7) / 8;
     plan.nsplit = 0;
@@ -1068,8 +1136,13 @@ int gemm_impl(const void* a, const void* sa, int64_t lda, const void* b, const v
   hipStream_t stm = (hipStream_t)stream;
 #define GEMM_LAUNCH(S) \
   launch<S>(A, SA, lda, B, SB, ldb, (int)M, (int)N, (int)K, cseg, lo, (int)r, plan, tiled, tnb, tn_blocks, pre, stm)
-  if (wide) GEMM_LAUNCH(Wide);
-  else GEMM_LAUNCH(Tall);
+  switch (shape) {
+    case ShapeId::kTall: GEMM_LAUNCH(Tall); break;
+    case ShapeId::kWide: GEMM_LAUNCH(Wide); break;
+    case ShapeId::kMid: GEMM_LAUNCH(Mid); break;
+    case ShapeId::kLow: GEMM_LAUNCH(Low); break;
+    case ShapeId::kSmall: GEMM_LAUNCH(Small); break;
+  }
 #undef GEMM_LAUNCH
   MX_CHECK_LAUNCH("mxfp8_gemm_nt");
   return MXFP8_OK;
@@ -1103,13 +1176,17 @@ extern "C" int mxfp8_gemm_nt_tn(const void* a, const void* sa, int64_t lda, cons
   int64_t nb = 0, ns = 0;
   int rc = tn_batch_tables("mxfp8_gemm_nt_tn", jobs, n_jobs, T_tn, K_tn, chunks, part, tnb, sa_tn, nb, ns);
   if (rc != MXFP8_OK) return rc;
-  MX_CHECK_ARG(nb + (M + 255) / 256 * (N / 128) + 8 < (1LL << 31), "mxfp8_gemm_nt_tn: too many workgroups");
+  MX_CHECK_ARG(nb + (M + 63) / 64 * (N / 64) + 8 < (1LL << 31), "mxfp8_gemm_nt_tn: too many workgroups");
   CSeg cs{};
   cs.n = 1;
   cs.ptr[0] = (uint16_t*)c;
   cs.ld[0] = ldc;
+  // the 8-wave shape does not carry the reductions: they get their own launch
+  const ShapeId shape = N > 0 && K > 0 ? pick_shape(M, N, K, cached_cus(), true, kUnfoldedTn) : ShapeId::kTall;
+  const bool fold = shape != ShapeId::kWide;
   rc = gemm_impl(a, sa, lda, b, sb, ldb, M, N, K, cs, lora_p, ld_p, lora_q, ld_q, r, alpha, layout, nullptr, 0, stream,
-                 tnb, nb);
+                 tnb, fold ? nb : 0, PreSum{}, (int)shape);
+  if (rc == MXFP8_OK && !fold) rc = tn_batch_launch(tnb, nb, (hipStream_t)stream, "mxfp8_gemm_nt_tn");
   if (rc != MXFP8_OK) return rc;
   return tn_sum_batch_launch(sa_tn, ns, (hipStream_t)stream, "mxfp8_gemm_nt_tn");
 }
@@ -1174,12 +1251,15 @@ extern "C" int mxfp8_gemm_nt_sum(const void* a, const void* sa, int64_t lda, con
   // find its flags already holding that id from the first and read P before this replay's sums.  A captured call
   // (or one on a stream whose capture state cannot be read) therefore sums P in a launch of its own, the same
   // bits, before the plain GEMM.
+  // The 8-wave shape has no summing workgroups either.
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess || cap != hipStreamCaptureStatusNone) {
+  const ShapeId shape = N > 0 && K > 0 ? pick_shape(M, N, K, cached_cus(), true, kUnfoldedSum) : ShapeId::kTall;
+  if (shape == ShapeId::kWide || hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess ||
+      cap != hipStreamCaptureStatusNone) {
     const int rc = mxfp8_sum_parts(part, n_parts, M * r, part_scale, lora_p, 1, stream);
     if (rc != MXFP8_OK) return rc;
     return gemm_impl(a, sa, lda, b, sb, ldb, M, N, K, cs, lora_p, r, lora_q, ld_q, r, alpha, layout, nullptr, 0,
-                     stream);
+                     stream, TnBatch{}, 0, PreSum{}, (int)shape);
   }
   unsigned long long* flags = presum_flags_on_current_device();
   if (!flags) return MXFP8_ERR_ARG;
@@ -1197,7 +1277,7 @@ extern "C" int mxfp8_gemm_nt_sum(const void* a, const void* sa, int64_t lda, con
   pre.wait_limit = wait_limit < 0 ? (1 << 20) : (int)std::min<int64_t>(wait_limit, 1 << 30);
   pre.scale = part_scale;
   return gemm_impl(a, sa, lda, b, sb, ldb, M, N, K, cs, lora_p, r, lora_q, ld_q, r, alpha, layout, nullptr, 0, stream,
-                   TnBatch{}, 0, pre);
+                   TnBatch{}, 0, pre, (int)shape);
 }
 
 extern "C" int mxfp8_gemm_nt_seg(const void* a, const void* sa, int64_t lda, const void* b, const void* sb,
@@ -1245,8 +1325,14 @@ extern "C" int mxfp8_gemm_swiglu_fwd(const void* a, const void* sa, const void* 
                    mx_aligned(xs, 16) && mx_aligned(bg, 16) && mx_aligned(bu, 16) && mx_aligned(ad, 16) &&
                    mx_aligned(gu, 16) && mx_aligned(q_h, 16) && mx_aligned(part, 16),
                "mxfp8_gemm_swiglu_fwd: misaligned buffer");
+  // Mid while its tiles run in one round (us, Tall / Mid, r = 16: M = 256, d_ffn 3584, K 1024 12.6 / 9.2; M = 512,
+  // d_ffn 2560, K 1536 14.9 / 11.1; in two rounds M = 1000, d_ffn 2560 16.6 / 17.0); the epilogue is most of the rest,
+  // and Wide is within 3% of Tall either way.
+  const int cus = cached_cus();
+  const bool mid = (M + Mid::kBM - 1) / Mid::kBM * (2 * N / Mid::kBN) <= cus;
   Plan plan;
-  make_plan<Tall>(M, 2 * N, K, cached_cus(), plan);
+  if (mid) make_plan<Mid>(M, 2 * N, K, cus, plan);
+  else make_plan<Tall>(M, 2 * N, K, cus, plan);
   SwEpi sw{(const uint16_t*)xs, (const uint16_t*)bg, (const uint16_t*)bu, (const uint16_t*)ad, s_g, s_u,
            (uint16_t*)gu, (uint8_t*)q_h, (uint8_t*)s_h, part, (int)N};
   CSeg cs{};
@@ -1258,8 +1344,13 @@ extern "C" int mxfp8_gemm_swiglu_fwd(const void* a, const void* sa, const void* 
 #define SWIGLU_LAUNCH(R, S)                                                                                        \
   gemm_kernel<R, S, kEpiSwiGluFwd><<<grid, S::kThreads, 0, stm>>>(A, SA, K, B, SB, K, (int)M, (int)(2 * N), (int)K, cs, \
                                                                   Lora{}, plan, tiled, sw, SwBwd{}, TnBatch{}, PreSum{})
-  if (r == 16) SWIGLU_LAUNCH(16, Tall);
-  else SWIGLU_LAUNCH(32, Tall);
+  if (mid) {
+    if (r == 16) SWIGLU_LAUNCH(16, Mid);
+    else SWIGLU_LAUNCH(32, Mid);
+  } else {
+    if (r == 16) SWIGLU_LAUNCH(16, Tall);
+    else SWIGLU_LAUNCH(32, Tall);
+  }
 #undef SWIGLU_LAUNCH
   MX_CHECK_LAUNCH("mxfp8_gemm_swiglu_fwd");
   return MXFP8_OK;

@@ -164,6 +164,8 @@ struct TnSumBatch {
 // the reduction and of the sum grids.  Returns MXFP8_OK, or MXFP8_ERR_ARG with the message set under `who`.
 int tn_batch_tables(const char* who, const mxfp8_lora_tn_job* jobs, int64_t n_jobs, int64_t T, int64_t K,
                     int64_t chunks, float* part, TnBatch& a, TnSumBatch& sa, int64_t& nb, int64_t& ns);
+// Host side (lora.hip): launch a batch filled by tn_batch_tables as a grid of its own.
+int tn_batch_launch(const TnBatch& a, int64_t nb, hipStream_t stm, const char* who);
 // Host side (lora.hip): launch the sums of a batch filled by tn_batch_tables.
 int tn_sum_batch_launch(const TnSumBatch& sa, int64_t ns, hipStream_t stm, const char* who);
 
