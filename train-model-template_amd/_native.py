@@ -5,12 +5,14 @@ HIP stream of the tensors' device, so launches stay asynchronous and ordered wit
 is no fallback: if the library is missing or does not match this module's ABI version, the first call raises.
 """
 import ctypes
+import importlib.util
 import os
 
 import torch
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmxfp8_mlp.so")
+HOST_PATH = os.path.join(_HERE, "_mxhost.so")
 ABI_VERSION = 14
 GEMM_A_TILED, GEMM_B_TILED, GEMM_WIDE, GEMM_C_FT, GEMM_B_PI = 1, 2, 4, 8, 16  # mxfp8_gemm_nt layout bits
 
@@ -104,10 +106,33 @@ def _check(rc, name):
         raise NativeError(f"{name} failed with code {rc}: {_lib.mxfp8_last_error().decode()}")
 
 
+_host = None
+
+
+def host():
+    """The native host module (csrc/host_path.cpp): allocation and launches of a hot call in one step."""
+    global _host
+    if _host is None:
+        load()
+        if not os.path.exists(HOST_PATH):
+            raise NativeError(f"{HOST_PATH} is not built: run `python -c 'import __graft_entry__ as g; g.build()'`")
+        spec = importlib.util.spec_from_file_location("_mxhost", HOST_PATH)
+        m = importlib.util.module_from_spec(spec)
+        spec.loader.exec_module(m)
+        if m.abi_version() != ABI_VERSION:
+            raise NativeError(f"{HOST_PATH}: built against ABI version {m.abi_version()}, expected {ABI_VERSION}")
+        m.set_error(NativeError)
+        _host = m
+    return _host
+
+
 _raw_stream = torch._C._cuda_getCurrentRawStream  # device index -> the current HIP stream, as an int
 
 
-def _stream(t):
+def stream_of(t, what="mxfp8"):
+    """The current stream of the tensor's device, as an int."""
+    if not t.is_cuda:
+        _gpu(t, what)
     return _raw_stream(t.get_device())
 
 

@@ -32,25 +32,40 @@ FOLD_TN = [os.environ.get("MXFP8_GROUP_FOLD_TN", "1") != "0"]
 STATS = {"gộp": 0, "gọi thẳng": 0}  # path counters, the reference's keys (grouped / called directly)
 
 
+_NONE = object()
+
+
+def _attr(m, name, *default):
+    """getattr(m, name, *default) of a module's parameter or submodule, looked up where nn.Module keeps them:
+    Module.__getattr__ is reached only after the ordinary lookup has failed, 0.5 us each time on the host."""
+    d = m.__dict__
+    for kind in ("_parameters", "_modules"):
+        v = d.get(kind, d).get(name, _NONE)
+        if v is not _NONE:
+            return v
+    return getattr(m, name, *default)
+
+
 def _part(m):
     """(base Linear, A, B, scaling) of a PEFT LoRA Linear; (m, None, None, 1.0) for a plain frozen Linear;
     None if the layer cannot be grouped (fused_linear.py:30-48)."""
-    base = getattr(m, "base_layer", None)
+    base = _attr(m, "base_layer", None)
     if base is None:
-        if type(m) is nn.Linear and m.bias is None and not m.weight.requires_grad:
+        if type(m) is nn.Linear and _attr(m, "bias") is None and not _attr(m, "weight").requires_grad:
             return m, None, None, 1.0
         return None
-    if base.bias is not None or base.weight.requires_grad or m.merged or m.disable_adapters:
+    if _attr(base, "bias") is not None or _attr(base, "weight").requires_grad or m.merged or m.disable_adapters:
         return None
-    ads = [a for a in m.active_adapters if a in m.lora_A]
+    lora_A = _attr(m, "lora_A")
+    ads = [a for a in m.active_adapters if a in lora_A]
     if len(ads) != 1:
         return None
     a = ads[0]
-    drop = m.lora_dropout[a]
-    if (a in getattr(m, "lora_variant", {}) or m.use_dora.get(a, False) or m.lora_B[a].bias is not None
+    drop, lora_B = _attr(m, "lora_dropout")[a], _attr(m, "lora_B")[a]
+    if (a in getattr(m, "lora_variant", ()) or m.use_dora.get(a, False) or _attr(lora_B, "bias") is not None
             or not (isinstance(drop, nn.Identity) or getattr(drop, "p", 1) == 0)):
         return None
-    return base, m.lora_A[a].weight, m.lora_B[a].weight, m.scaling[a]
+    return base, _attr(lora_A[a], "weight"), _attr(lora_B, "weight"), m.scaling[a]
 
 
 # bf16 copies of the LoRA A/B parameters (fp32) and the concatenated S matrix, made once per training step
@@ -300,7 +315,6 @@ def _fwd_merged(spec, Bs, xS, codes, T, dt, skey):
         Q = forms.Q
     else:
         Q = _cast(skey + ("qcat", tuple(spec.mx), rp), block_diagonal_b)
-    outs = [torch.empty((T, n), dtype=dt, device=xS.device) for n in widths]
     # every layer with an adapter of one width: each output tile takes the rank-width window of xS and Q at its
     # layer's own columns (the rest of its Q row is zero) instead of all rp columns
     ranks = {sl.width for sl in slots if sl is not None}
@@ -308,7 +322,13 @@ def _fwd_merged(spec, Bs, xS, codes, T, dt, skey):
         cols = dict(lora_cols=[sl.col for sl in slots], r=ranks.pop())
     else:
         cols = {}
-    mxfp8.mx_mm_seg(codes[0], codes[1], op[0], op[1], outs, lora=(xS, Q), alpha=alpha, layout=3, m=T, **cols)
+    if mxfp8.GEMM_EVENTS is None:
+        import _native
+        outs = _native.host().gemm_seg(codes[0], codes[1], op[0], op[1], widths, xS, Q, alpha, 3, T,
+                                       cols.get("lora_cols", ()), cols.get("r", 0), _native.stream_of(xS))
+    else:
+        outs = [torch.empty((T, n), dtype=dt, device=xS.device) for n in widths]
+        mxfp8.mx_mm_seg(codes[0], codes[1], op[0], op[1], outs, lora=(xS, Q), alpha=alpha, layout=3, m=T, **cols)
     return dict(zip(spec.mx, outs))
 
 
@@ -480,20 +500,18 @@ def _fused_bwd_plan(spec, flat, dt, need_x):
 
 
 def _lora_bwd_batchable(spec, flat, xS):
-    """The adapter slots of the group's MX layers when their lora_bwd calls can run as one batch: 2..8 MX layers,
+    """The adapter slots of the group's MX layers when their lora_bwd calls can run as one: 1..8 MX layers,
     each with an adapter of one common rank 16 or 32 whose xS columns the kernel reads with 16-byte loads, and
     row-contiguous, 16-byte aligned dy; else None."""
     import _native
-    slots = [spec.adapter(i) for i in spec.mx]
-    if not 2 <= len(slots) <= _native.LORA_BWD_MAX_JOBS or any(sl is None for sl in slots):
+    slots = [spec._adapter.get(i) for i in spec.mx]
+    if not 1 <= len(slots) <= _native.LORA_BWD_MAX_JOBS or slots[0] is None or slots[0].width not in (16, 32):
         return None
-    if len({sl.width for sl in slots}) != 1 or slots[0].width not in (16, 32):
+    if not _vec_ok(xS):  # and its slot columns: they start at multiples of 8 values
         return None
-    if not all(_vec_ok(xS[:, sl.cols]) for sl in slots):
-        return None
-    if not all(flat[i].stride(1) == 1 and flat[i].stride(0) % 8 == 0 and flat[i].data_ptr() % 16 == 0
-               for i in spec.mx):
-        return None
+    for sl, i in zip(slots, spec.mx):
+        if sl is None or sl.width != slots[0].width or sl.col % 8 or not _vec_ok(flat[i]):
+            return None
     return slots
 
 
@@ -518,23 +536,20 @@ def _fused_backward(spec, skey, x2, xS, S, Bs, flat, plan, need_x, dt):
         dS[:, n_cols:].zero_()
     grads = [None] * (2 * len(spec.adapters))
     q = sbuf = None
-    if need_x:
+    tile = 0
+    batch = T > 0 and _lora_bwd_batchable(spec, flat, xS)
+    if batch:
+        # every MX layer's lora_bwd (mxfp8.lora_bwd, lora_bwd_batch) in one call: one launch and one of its sums
+        import _native
+        q, sbuf, dbs = _native.host().group_lora_bwd([flat[i] for i in spec.mx], xS, [Bs[sl.index] for sl in batch],
+                                                     [sl.col for sl in batch], [sl.scale for sl in batch], dS, need_x,
+                                                     _native.stream_of(x2))
+        for sl, db in zip(batch, dbs):
+            grads[2 * sl.index + 1] = db
+    elif need_x:
         n_mx = sum(flat[i].shape[1] for i in spec.mx)
         q = torch.empty((T, n_mx), dtype=mxfp8.F8, device=dev)
         sbuf = torch.empty(_cdiv(T, 128) * (n_mx // 128) * 512, dtype=torch.uint8, device=dev)
-    tile = 0
-    batch = _lora_bwd_batchable(spec, flat, xS)
-    if batch:
-        # every MX layer's lora_bwd in one launch (mxfp8_lora_bwd_batch)
-        offs, t = [], 0
-        for i in spec.mx:
-            offs.append(t)
-            t += flat[i].shape[1] // 128
-        dbs = mxfp8.lora_bwd_batch([flat[i] for i in spec.mx], [xS[:, sl.cols] for sl in batch],
-                                   [Bs[sl.index] for sl in batch], [sl.scale for sl in batch],
-                                   [dS[:, sl.cols] for sl in batch], q=q, s=sbuf, col_tile_offs=offs)
-        for sl, db in zip(batch, dbs):
-            grads[2 * sl.index + 1] = db
     for i in (() if batch else spec.mx):
         dy = flat[i] if flat[i].stride(1) == 1 else flat[i].contiguous()
         sl = spec.adapter(i)

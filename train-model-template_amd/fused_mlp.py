@@ -24,6 +24,7 @@ Every kernel of the path is hand-written HIP (libmxfp8_mlp.so, _native.py): the 
 the quantizer (xs with MX(x), dxd with MX(dy)), the GEMM epilogues (y, dx) and the token-reduction kernel
 (dB_d, dA); no BLAS or elementwise torch kernel runs inside a step.
 """
+import functools
 import os
 import types
 
@@ -83,19 +84,24 @@ def _bwd_grid(T, N, R, wide=False):
     so the time goes as rounds x (SB/32 row blocks x column passes); pick the least of that, then the fewest
     partial-sum bytes (per super-block dB / dA_d partials; the dxa partials are one per 128 (wide: 256) columns
     whatever the grid; the trade-off of fused_mlp.py:218-232)."""
-    tpad = _cdiv(T, 128) * 128
-    cap = _n_cu() * (1 if wide else 2)
+    return _grid_search(_cdiv(T, 128), N, R, wide, _n_cu() * (1 if wide else 2))
+
+
+@functools.lru_cache(maxsize=1024)
+def _grid_search(tiles, N, R, wide, cap):
+    """_bwd_grid's choice among CG and, for each count of super-blocks, the smallest SB that gives it (a larger one
+    is more work for the same count).  A pure function of its arguments, kept for the sizes seen last: trying every
+    multiple of 128 rows took 0.13 ms of host time at T = 4096 and 0.7 ms at T = 10752."""
     cols = 256 if wide else 128
     best = None
     for cg in [cols * d for d in _divisors(N // cols)]:
-        ncg = N // cg
-        for sb in range(128, tpad + 128, 128):
-            nsb = _cdiv(tpad, sb)
-            work = _cdiv(nsb * ncg, cap) * (sb // 32) * (cg // cols)
-            partial = nsb * N * R * 3 * 4
-            key = (work, partial)
+        ncg, t = N // cg, 1
+        while t <= tiles:  # t: 128-row tiles per super-block
+            nsb = _cdiv(tiles, t)
+            key = (_cdiv(nsb * ncg, cap) * (t * 4) * (cg // cols), nsb * N * R * 3 * 4)
             if best is None or key < best[0]:
-                best = (key, sb, cg)
+                best = (key, t * 128, cg)
+            t = tiles + 1 if nsb == 1 else _cdiv(tiles, nsb - 1)  # the next count's smallest
     return best[1], best[2]
 
 
@@ -183,19 +189,15 @@ def mlp_bwd(gu, xs, dhm, dxd, bg, bu, ad, s_g, s_u, need_q, dgu_out=None, tiled=
     return q, s, dxa, dbg, dbu, dad
 
 
+_FORMS = ("S", "ST", "bg", "bu", "bgT", "buT", "ad", "adT", "bd", "bdT")  # in _native.host().mlp_forms' order
+
+
 def _prep(Ag, Bg, Au, Bu, Ad, Bd, dt):
     """The step's bf16 forms of the LoRA weights (fused_mlp.py:272-276 _cast copies, plus the transposed copies
     the kernels index), from one kernel; cached per step like fused_linear._cast."""
     def make():
-        dev = Ag.device
-        R, K = Ag.shape
-        N = Bg.shape[0]
-        e = lambda *sh: torch.empty(sh, dtype=torch.bfloat16, device=dev)  # noqa: E731
-        out = dict(S=e(2 * R, K), ST=e(K, 2 * R), bg=e(N, R), bu=e(N, R), bgT=e(R, N), buT=e(R, N), ad=e(R, N),
-                   adT=e(N, R), bd=e(K, R), bdT=e(R, K))
-        f = lambda t: t.detach().float().contiguous()  # noqa: E731
-        _native.lora_prep(f(Ag), f(Au), f(Bg), f(Bu), f(Ad), f(Bd), out)
-        return types.SimpleNamespace(**out)
+        return types.SimpleNamespace(**dict(zip(_FORMS, _native.host().mlp_forms(
+            (Ag, Bg, Au, Bu, Ad, Bd), _native.stream_of(Ag, "mxfp8_lora_prep")))))
     return _cast((("lora_prep", id(Ag), id(Au), id(Bg), id(Bu), id(Ad), id(Bd)), dt), make)
 
 
@@ -231,6 +233,17 @@ def _forms_of_saved(S, bg, bu, ad, bd, dt):
 _LAYOUT_FT = _native.GEMM_A_TILED | _native.GEMM_B_TILED | _native.GEMM_C_FT
 
 
+def _fwd_in_one_call(down, need_out):
+    """The forward's launches come from one call of the native host module: the default switches, and no GEMM
+    events to record.  The code it stands for follows it in _MLP.forward."""
+    return (FUSED_EPILOGUE[0] and FOLD_SUM[0] and B_PI[0] and mxfp8.GEMM_EVENTS is None
+            and (not need_out or "_mx_wp_tl" in down.__dict__))
+
+
+def _bwd_in_one_call():
+    return FOLD_TN[0] and B_PI[0] and not FUSED_BWD_EPILOGUE[0] and mxfp8.GEMM_EVENTS is None
+
+
 class _MLP(torch.autograd.Function):
     """fused_mlp.py:262-336."""
 
@@ -248,8 +261,16 @@ class _MLP(torch.autograd.Function):
         # one read of x2: its MX operand (MX-tiled codes, the GEMM's operand layout; same codes and scales as
         # mx_quant) and xs = bf16(x2 · Sᵀ) [T, 2R] = xa_gate | xa_up, with the zero-padded transpose the backward
         # kernel reads
-        q, sc, xs, _ = mxfp8.mx_quant_lora(x2, S, out_t=False)  # 2R in {32, 64} (r in {16, 32}, _r_ok)
-        if need_out and FUSED_EPILOGUE[0]:
+        one = _fwd_in_one_call(down, need_out)
+        if not one:
+            q, sc, xs, _ = mxfp8.mx_quant_lora(x2, S, out_t=False)  # 2R in {32, 64} (r in {16, 32}, _r_ok)
+        if one and need_out:  # every launch of the next two branches and of the down GEMM below
+            y, xs, gu = _native.host().mlp_forward(
+                x2, S, bg, bu, ad, bd, hold.wf_tl, hold.wfs, down._mx_wp_tl, down._mx_wps, s_g, s_u, s_d,
+                _native.GEMM_NT_SUM_MAX, _native.stream_of(x2))
+        elif one:
+            xs, gu = _native.host().mlp_graph(x2, S, hold.w_tl, hold.ws, hold.n, _native.stream_of(x2))
+        elif need_out and FUSED_EPILOGUE[0]:
             # one launch: gu = gate | up [T, 2N] (fused-tile layout, the saved tensor) and, in the GEMM's epilogue,
             # the LoRA-B of gate and up, h = silu(g)·u, MX(h) and the per-tile xS_down partials
             gu, qh, sh, part = mxfp8.swiglu_gemm(q, sc, hold, xs, bg, bu, ad, s_g, s_u, T)
@@ -265,7 +286,7 @@ class _MLP(torch.autograd.Function):
             del q, sc
             if need_out:
                 qh, sh, xsd = mlp_fwd(gu, xs, bg, bu, ad, s_g, s_u, True, tiled=True, gu_ft=True)
-        if need_out:
+        if need_out and not one:
             # y = bf16(bf16(MX(h)·W_downᵀ) + s_d · xS_down · B_dᵀ): the addmm_ of fused_mlp.py:284 in the epilogue
             w, ws, lay = ((down._mx_wp_tl, down._mx_wps, 3 | _native.GEMM_B_PI)
                           if B_PI[0] and "_mx_wp_tl" in down.__dict__ else (down._mx_w_tl, down._mx_ws, 3))
@@ -274,7 +295,7 @@ class _MLP(torch.autograd.Function):
             else:
                 y = mxfp8.mx_mm(qh, sh, w, ws, lora=(xsd, bd), alpha=s_d, layout=lay, m=T)
             del qh, sh, xsd, part
-        else:  # graph only (checkpoint recompute / prefix backward): nobody reads y
+        if not need_out:  # graph only (checkpoint recompute / prefix backward): nobody reads y
             STATS["bỏ đầu ra"] = STATS.get("bỏ đầu ra", 0) + 1
             y = x2.new_empty(x2.shape[0], down.out_features)
         # the reference's saved set, the same in both modes (non-reentrant checkpointing compares metadata on
@@ -299,6 +320,19 @@ class _MLP(torch.autograd.Function):
             dy2 = dy2.contiguous()
         T, N = dy2.shape[0], hold.n
         lw = _forms_of_saved(S, bg, bu, ad, bd, dt)
+        ag_dt, au_dt, bd_dt = ctx.pdt
+        fp32_a = ag_dt == au_dt == torch.float32
+        if _bwd_in_one_call():  # every launch of the code below
+            wide = WIDE_BWD[0] and N % 256 == 0
+            SB, CG = _bwd_grid(T, N, R, wide)
+            LAST["bwd"] = dict(SB=SB, CG=CG, nsb=_cdiv(_cdiv(T, 128) * 128, SB), ncg=N // CG, wide=wide)
+            dx, dA, dB_g, dB_u, dA_d, dB_d = _native.host().mlp_backward(
+                dy2, x2, xs, gu, (S, lw.ST, bg, bu, lw.bgT, lw.buT, ad, lw.adT, bd, lw.bdT),
+                *mxfp8.dgrad_rows_operand(down), hold.wtp_tl, hold.wtps, s_g, s_u, s_d, SB, CG, wide, need_x, fp32_a,
+                bd_dt == torch.float32, _native.stream_of(dy2))
+            if need_x:
+                dx = dx.view(*lead, K).to(xdt)
+            return _wanted(ctx, dx, (dA[:R], dB_g, dA[R:], dB_u, dA_d, dB_d))
         # one read of dy2: its MX operand and dxd = bf16(bf16(dy2 · bd) · s_d) [T, R] with its zero-padded transpose,
         # and, from the same launch, xsT, the backward kernel's operand form of xs (zero-padded transpose)
         qd, sd, dxd, dxdT, xsT = mxfp8.mx_quant_lora_tp(dy2, lw.bdT, xs, scale=s_d)
@@ -333,8 +367,6 @@ class _MLP(torch.autograd.Function):
         # parameter's dtype anyway (bf16 -> fp32 is exact, so .grad is bit-identical), and the kernel writing the
         # fp32 holder directly saves those cast kernels (about 23 us per step at the headline shape).  Both in one
         # launch (and their chunk sums in one more): dB_d = bf16(bf16(dyᵀ xsd) s_d) and dA = bf16(dxaᵀ · x2)
-        ag_dt, au_dt, bd_dt = ctx.pdt
-        fp32_a = ag_dt == au_dt == torch.float32
         chunks = _native.lora_tn_chunks(T, K)
         part = torch.empty(chunks * 3 * R * K, dtype=torch.float32, device=dy2.device)
         dB_d = torch.empty((K, R), dtype=torch.float32 if bd_dt == torch.float32 else dt, device=dy2.device)
@@ -358,9 +390,12 @@ class _MLP(torch.autograd.Function):
                 dx = mxfp8.mx_mm(qg, sg, w, ws, lora=(dxa, lw.ST), alpha=1.0, layout=lay, m=T)
             del qg, sg
             dx = dx.view(*lead, K).to(xdt)
-        grads = [dA[:R], dB_g, dA[R:], dB_u, dA_d, dB_d]
-        ws_in = ctx.needs_input_grad[3:]
-        return (dx, None, None, *[g if ws_in[k] else None for k, g in enumerate(grads)])
+        return _wanted(ctx, dx, (dA[:R], dB_g, dA[R:], dB_u, dA_d, dB_d))
+
+
+def _wanted(ctx, dx, grads):
+    ws_in = ctx.needs_input_grad[3:]
+    return (dx, None, None, *[g if ws_in[k] else None for k, g in enumerate(grads)])
 
 
 def _r_ok(r):

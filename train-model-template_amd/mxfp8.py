@@ -43,11 +43,9 @@ def mx_quant(x2d):
     Replaces the Triton _quant_kernel launch of mxfp8.py:78-86."""
     R, K = x2d.shape
     assert x2d.dtype == torch.bfloat16 and x2d.is_contiguous() and K % 128 == 0, (x2d.dtype, x2d.shape)
-    q = torch.empty((R, K), dtype=F8, device=x2d.device)
-    s = torch.empty(scale_numel(R, K), dtype=torch.uint8, device=x2d.device)
-    if R:
-        _native.quant_rows(x2d, q, s)
-    return q, s.view(E8)
+    if R == 0:
+        return torch.empty((0, K), dtype=F8, device=x2d.device), torch.empty(0, dtype=E8, device=x2d.device)
+    return _native.host().quant_rows(x2d, _native.stream_of(x2d, "mxfp8_quant_rows"))
 
 
 def tiled_rows(R):
@@ -66,11 +64,9 @@ def mx_quant_tiled(x2d):
     bytes; pass layout bits to mx_mm.  No reference counterpart (an internal layout of the fused path)."""
     R, K = x2d.shape
     assert x2d.dtype == torch.bfloat16 and x2d.stride(1) == 1 and K % 128 == 0, (x2d.dtype, x2d.shape)
-    q = torch.empty((tiled_rows(R), K), dtype=F8, device=x2d.device)
-    s = torch.empty(scale_numel(R, K), dtype=torch.uint8, device=x2d.device)
-    if R:
-        _native.quant_tiled(x2d, q, s)
-    return q, s.view(E8)
+    if R == 0:
+        return torch.empty((0, K), dtype=F8, device=x2d.device), torch.empty(0, dtype=E8, device=x2d.device)
+    return _native.host().quant_tiled(x2d, _native.stream_of(x2d, "mxfp8_quant_tiled"))
 
 
 def mx_quant_lora(x2d, w, scale=1.0, out_t=True):
@@ -78,14 +74,7 @@ def mx_quant_lora(x2d, w, scale=1.0, out_t=True):
     rp in {16, 32, 64}: -> (q, s, out [R, rp], outT [rp, ceil(R/128)*128] zero-padded, or None)."""
     R, K = x2d.shape
     assert x2d.dtype == torch.bfloat16 and x2d.stride(1) == 1 and K % 128 == 0 and R > 0, (x2d.dtype, x2d.shape)
-    rp = w.shape[0]
-    dev = x2d.device
-    q = torch.empty((tiled_rows(R), K), dtype=F8, device=dev)
-    s = torch.empty(scale_numel(R, K), dtype=torch.uint8, device=dev)
-    out = torch.empty((R, rp), dtype=torch.bfloat16, device=dev)
-    outT = torch.empty((rp, _cdiv(R, 128) * 128), dtype=torch.bfloat16, device=dev) if out_t else None
-    _native.quant_lora(x2d, q, s, w, out, scale=scale, outT=outT)
-    return q, s.view(E8), out, outT
+    return _native.host().quant_lora(x2d, w, scale, out_t, _native.stream_of(x2d, "mxfp8_quant_lora"))
 
 
 def mx_quant_lora_tp(x2d, w, tx, scale=1.0):
@@ -115,10 +104,9 @@ def res_lora(x, y, xa, B, scale):
     assert x.dtype == y.dtype == xa.dtype == B.dtype == torch.bfloat16 and x.is_contiguous() and y.is_contiguous()
     assert B.is_contiguous() and xa.stride(1) == 1 and B.shape == (N, xa.shape[1]) and xa.shape[0] == T
     assert xa.shape[1] in (16, 32), "res_lora: LoRA rank must be 16 or 32"
-    out = torch.empty_like(x)
-    if T:
-        _native.res_lora(x, y, xa, B, out, scale)
-    return out
+    if T == 0:
+        return torch.empty_like(x)
+    return _native.host().res_lora(x, y, xa, B, scale, _native.stream_of(x, "mxfp8_res_lora"))
 
 
 def lora_bwd(dy, xa=None, B=None, scale=1.0, q=None, s=None, col_tile_off=0, dxa_out=None):
@@ -269,15 +257,21 @@ def mx_mm(q, s, wq, ws, out=None, lora=None, alpha=1.0, layout=0, m=None):
     N = wq.shape[0]
     assert wq.shape[1] == K and q.stride(1) == 1 and wq.stride(1) == 1, (q.shape, wq.shape)
     assert not (layout & 1) or q.shape[0] == tiled_rows(M), (q.shape, M)
-    if out is None:
+    wide = layout & _native.GEMM_WIDE  # takes a workspace
+    if out is None and (wide or not M):
         out = torch.empty((ft_rows(M) if layout & 8 else M, N), dtype=torch.bfloat16, device=q.device)
     if M:
         ev = GEMM_EVENTS
         if ev is not None:
             e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
             e0.record()
-        _native.gemm_nt(q, s, q.stride(0), wq, ws, wq.stride(0), M, N, K, out, lora=lora, alpha=alpha,
-                        layout=layout)
+        if wide:
+            _native.gemm_nt(q, s, q.stride(0), wq, ws, wq.stride(0), M, N, K, out, lora=lora, alpha=alpha,
+                            layout=layout)
+        else:
+            P, Q = (None, None) if lora is None else lora
+            out = _native.host().gemm(q, s, wq, ws, out, P, Q, alpha, layout, M,
+                                      _native.stream_of(q, "mxfp8_gemm_nt"))
         if ev is not None:
             e1.record()
             ev.append((e0, e1, 2 * M * N * K))
@@ -317,13 +311,12 @@ def mx_mm_tn(q, s, wq, ws, lora, alpha, layout, m, tn_jobs, part):
     N = wq.shape[0]
     assert wq.shape[1] == K and q.stride(1) == 1 and wq.stride(1) == 1, (q.shape, wq.shape)
     assert not (layout & 1) or q.shape[0] == tiled_rows(M), (q.shape, M)
-    out = torch.empty((ft_rows(M) if layout & 8 else M, N), dtype=torch.bfloat16, device=q.device)
     ev = GEMM_EVENTS
     if ev is not None:
         e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
         e0.record()
-    _native.gemm_nt_tn(q, s, q.stride(0), wq, ws, wq.stride(0), M, N, K, out, lora, tn_jobs, part, alpha=alpha,
-                       layout=layout)
+    out = _native.host().gemm_tn(q, s, wq, ws, lora[0], lora[1], alpha, layout, M, tn_jobs, part,
+                                 _native.stream_of(q, "mxfp8_gemm_nt_tn"))
     if ev is not None:
         e1.record()
         ev.append((e0, e1, 2 * M * N * K))
