@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define MXFP8_MLP_ABI_VERSION 14
+#define MXFP8_MLP_ABI_VERSION 15
 #define MXFP8_OK 0
 #define MXFP8_ERR_ARG (-1)
 /* mxfp8_gemm_nt layout bits */
@@ -308,9 +308,11 @@ int64_t mxfp8_lora_bwd_batch_chunks(int64_t T, int64_t n_total);
  * as in mxfp8_lora_bwd, shared by the jobs.  Replaces the per-layer lora_bwd calls of the grouped backward
  * (/root/reference/scripts/fused_linear.py:219-259).  n_jobs <= MXFP8_LORA_BWD_MAX_JOBS, r in {16, 32}.
  * d(xa) is the same bits as mxfp8_lora_bwd's; dB is summed over other row chunks (fp32 rounding).
+ * q_tiled 1: the codes in the MX-tiled layout of mxfp8_quant_tiled (q holds ceil(T/16)*16 rows of ld_q columns, ld_q a
+ * multiple of 128; rows past T are not written), the layout the dx GEMM streams; 0: row-major with row stride ld_q.
  */
 int mxfp8_lora_bwd_batch(const mxfp8_lora_bwd_job* jobs, int64_t n_jobs, int64_t T, int64_t r, void* q, int64_t ld_q,
-                         void* s, int64_t s_col_tiles, void* stream);
+                         void* s, int64_t s_col_tiles, int64_t q_tiled, void* stream);
 
 /*
  * out [C, Tpad] bf16 = xᵀ of x [T, C] bf16 (row stride ld_x, 16-byte aligned rows), zero in columns T..Tpad-1.

@@ -13,7 +13,7 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libmxfp8_mlp.so")
 HOST_PATH = os.path.join(_HERE, "_mxhost.so")
-ABI_VERSION = 14
+ABI_VERSION = 15
 GEMM_A_TILED, GEMM_B_TILED, GEMM_WIDE, GEMM_C_FT, GEMM_B_PI = 1, 2, 4, 8, 16  # mxfp8_gemm_nt layout bits
 
 _i64, _ptr, _f32, _int = ctypes.c_int64, ctypes.c_void_p, ctypes.c_float, ctypes.c_int
@@ -56,7 +56,7 @@ SIGNATURES = {
     "mxfp8_lora_bwd": [_ptr, _i64, _i64, _i64, _ptr, _i64, _ptr, _i64, _i64, _ptr, _i64, _ptr, _i64, _f32, _ptr, _i64,
                        _ptr, _ptr, _ptr, _ptr],
     "mxfp8_lora_bwd_batch_chunks": [_i64, _i64],
-    "mxfp8_lora_bwd_batch": [_ptr, _i64, _i64, _i64, _ptr, _i64, _ptr, _i64, _ptr],
+    "mxfp8_lora_bwd_batch": [_ptr, _i64, _i64, _i64, _ptr, _i64, _ptr, _i64, _i64, _ptr],
     "mxfp8_lora_tn": [_ptr, _i64, _i64, _i64, _ptr, _i64, _i64, _ptr, _f32, _i64, _i64, _ptr, _ptr],
     "mxfp8_lora_tn_batch": [_ptr, _i64, _i64, _i64, _i64, _ptr, _ptr],
     "mxfp8_gemm_nt_sum": [_ptr, _ptr, _i64, _ptr, _ptr, _i64, _i64, _i64, _i64, _ptr, _i64, _ptr, _i64, _f32, _ptr,
@@ -446,7 +446,7 @@ def lora_bwd_batch(jobs, T, r, q, s):
     arr = (LoraBwdJob * len(table))(*table)
     call("mxfp8_lora_bwd_batch", ctypes.cast(arr, _ptr), len(table), T, r, _p(q) if q is not None else None,
          q.stride(0) if q is not None else 0, _p(s) if s is not None else None,
-         q.shape[1] // 128 if q is not None else 0, like=jobs[0][0])
+         q.shape[1] // 128 if q is not None else 0, 0, like=jobs[0][0])
 
 
 class PackJob(ctypes.Structure):

@@ -173,8 +173,9 @@ Tensor res_lora(const Tensor& x, const Tensor& y, const Tensor& xa, const Tensor
   return out;
 }
 
-// mxfp8.lora_bwd / lora_bwd_batch of a group's MX layers (one common rank): codes of every dy side by side in q, each
-// layer's d(xa) in its columns of dS, and the layers' dB.
+// mxfp8.lora_bwd / lora_bwd_batch of a group's MX layers (one common rank): codes of every dy side by side in q (in the
+// MX-tiled layout, the same bytes in the order that the dx GEMM streams), each layer's d(xa) in its columns of dS, and
+// the layers' dB.
 std::tuple<OptT, OptT, std::vector<Tensor>> group_lora_bwd(const std::vector<Tensor>& dys, const Tensor& xS,
                                                            const std::vector<Tensor>& Bs,
                                                            const std::vector<int64_t>& cols,
@@ -187,10 +188,10 @@ std::tuple<OptT, OptT, std::vector<Tensor>> group_lora_bwd(const std::vector<Ten
   for (const auto& d : dys) sum_n += d.size(1);
   OptT q, s;
   if (need_q) {
-    q = empty({T, sum_n}, kF8, dys[0]);
+    q = empty({tiled_rows(T), sum_n}, kF8, dys[0]);
     s = empty({scale_numel(T, sum_n)}, kE8, dys[0]);
   }
-  const int64_t chunks = n == 1 ? mxfp8_lora_bwd_chunks(T, sum_n) : mxfp8_lora_bwd_batch_chunks(T, sum_n);
+  const int64_t chunks = mxfp8_lora_bwd_batch_chunks(T, sum_n);
   Arena a;
   int64_t pdx[MXFP8_LORA_BWD_MAX_JOBS], pdb[MXFP8_LORA_BWD_MAX_JOBS];
   std::vector<Tensor> dbs;
@@ -209,23 +210,16 @@ std::tuple<OptT, OptT, std::vector<Tensor>> group_lora_bwd(const std::vector<Ten
   a.make(dys[0]);
   auto* xs = static_cast<uint16_t*>(xS.data_ptr());
   auto* ds = static_cast<uint16_t*>(dS.data_ptr());
-  if (n == 1) {
-    ok(mxfp8_lora_bwd(ptr(dys[0]), T, sum_n, dys[0].stride(0), ptr(q), need_q ? sum_n : 0, ptr(s),
-                      need_q ? sum_n / 128 : 0, 0, xs + cols[0], xS.stride(0), ptr(Bs[0]), R, (float)scales[0],
-                      ds + cols[0], dS.stride(0), fptr(dbs[0]), a.f(pdx[0]), a.f(pdb[0]), stm(stream)),
-       "mxfp8_lora_bwd");
-  } else {
-    mxfp8_lora_bwd_job jobs[MXFP8_LORA_BWD_MAX_JOBS];
-    int64_t tile = 0;
-    for (int64_t k = 0; k < n; ++k) {
-      const int64_t N = dys[k].size(1);
-      jobs[k] = {ptr(dys[k]), N,         dys[k].stride(0), need_q ? tile : 0, xs + cols[k], xS.stride(0), ptr(Bs[k]),
-                 (float)scales[k], ds + cols[k], dS.stride(0), fptr(dbs[k]), a.f(pdx[k]), a.f(pdb[k])};
-      tile += N / 128;
-    }
-    ok(mxfp8_lora_bwd_batch(jobs, n, T, R, ptr(q), need_q ? sum_n : 0, ptr(s), need_q ? sum_n / 128 : 0, stm(stream)),
-       "mxfp8_lora_bwd_batch");
+  mxfp8_lora_bwd_job jobs[MXFP8_LORA_BWD_MAX_JOBS];
+  int64_t tile = 0;
+  for (int64_t k = 0; k < n; ++k) {
+    const int64_t N = dys[k].size(1);
+    jobs[k] = {ptr(dys[k]), N,         dys[k].stride(0), need_q ? tile : 0, xs + cols[k], xS.stride(0), ptr(Bs[k]),
+               (float)scales[k], ds + cols[k], dS.stride(0), fptr(dbs[k]), a.f(pdx[k]), a.f(pdb[k])};
+    tile += N / 128;
   }
+  ok(mxfp8_lora_bwd_batch(jobs, n, T, R, ptr(q), need_q ? sum_n : 0, ptr(s), need_q ? sum_n / 128 : 0, need_q, stm(stream)),
+     "mxfp8_lora_bwd_batch");
   return {q, s, dbs};
 }
 
@@ -370,7 +364,7 @@ PYBIND11_MODULE(_mxhost, m) {
     Py_XDECREF(g_error);
     g_error = e.ptr();
   });
-  m.def("abi_version", &mxfp8_abi_version);
+  m.def("abi_version", [] { return MXFP8_MLP_ABI_VERSION; });
   m.def("quant_rows", &quant_rows);
   m.def("quant_tiled", &quant_tiled);
   m.def("quant_lora", &quant_lora);

@@ -418,7 +418,8 @@ __device__ __forceinline__ void lora_bwd_body(const uint16_t* __restrict__ dy, i
                                               const uint16_t* __restrict__ xa, int64_t ld_xa,
                                               const uint16_t* __restrict__ B, float* __restrict__ part_dxa,
                                               float* __restrict__ part_db, uint16_t* __restrict__ dxa, int64_t ld_dxa,
-                                              float scale, const int bx, const int by, const int ny) {
+                                              float scale, const int bx, const int by, const int ny,
+                                              const bool tiled) {
   constexpr int kTileB = 32 * 256;         // one block of one wave: 32 rows x 128 bf16
   constexpr int kRedB = kLora ? 4 * 128 * 17 * 4 : 0;  // end-of-kernel dB exchange: [wave][column][16 ρ + 1]
   constexpr int kXaL = kLora ? R / 16 : 0;  // 16-byte xa pieces per lane per block
@@ -534,12 +535,18 @@ __device__ __forceinline__ void lora_bwd_body(const uint16_t* __restrict__ dy, i
       // the block's codes as whole 128-byte row pieces: lane l takes row 8 j + l / 8, chunk l % 8 (rows past T hold
       // row T - 1's codes and store them again); the four scale bytes of a row are one word of the 128 x 4 tile
       // (lanes l and l + 32 store the same word)
-      uint8_t* qrow = q + (int64_t)col_tile_off * 128 + c0 + (lane & 7) * 16;
+      // Tiled is what the dx GEMM reads: with row-major codes its 64-byte row pieces use half of each line per request
+      // (q|k|v dx with its reduction at T = 10752, K = 3072: 107 -> 92 us, o_proj's, K = 2048: 73 -> 64; this kernel the
+      // same within 1 us).  In the MX-tiled layout (ld_q = its columns) the block is four contiguous 1 KB blocks of it: store j takes row
+      // half j / 2 and column half j % 2, lane l row l / 4 of it at 16-byte position l % 4.
+      const int64_t qc = (int64_t)col_tile_off * 128 + c0;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
-        const int rr = 8 * j + (lane >> 3);
-        const uint4 cw = *reinterpret_cast<const uint4*>(qtile[w] + rr * 128 + (((lane & 7) ^ (rr & 7)) << 4));
-        store_codes<MX_NT_FUSED>(qrow + (int64_t)min(rb + rr, T - 1) * ld_q, cw);
+        const int rr = tiled ? 16 * (j >> 1) + (lane >> 2) : 8 * j + (lane >> 3);
+        const int ch = tiled ? 4 * (j & 1) + ((lane & 3) ^ ((lane >> 4) & 3)) : lane & 7;
+        const uint4 cw = *reinterpret_cast<const uint4*>(qtile[w] + rr * 128 + ((ch ^ (rr & 7)) << 4));
+        const int64_t mq = min(rb + rr, T - 1);
+        store_codes<MX_NT_FUSED>(q + (tiled ? tiled_offset(mq, qc + ch * 16, ld_q) : mq * ld_q + qc + ch * 16), cw);
       }
       store_codes<MX_NT_FUSED>(s + (((int64_t)(m >> 7) * s_col_tiles + col_tile_off + (c0 >> 7)) << 9) +
                                    (m & 31) * 16 + ((m & 127) >> 5) * 4,
@@ -633,7 +640,7 @@ __global__ __launch_bounds__(256, 2) void lora_bwd_kernel(const uint16_t* __rest
                                                           float* __restrict__ part_dxa, float* __restrict__ part_db,
                                                           uint16_t* __restrict__ dxa, int64_t ld_dxa, float scale) {
   lora_bwd_body<R, kQuant, kLora>(dy, ld_dy, T, N, Tpad, chunk, q, ld_q, s, s_col_tiles, col_tile_off, xa, ld_xa, B,
-                                  part_dxa, part_db, dxa, ld_dxa, scale, blockIdx.x, blockIdx.y, gridDim.y);
+                                  part_dxa, part_db, dxa, ld_dxa, scale, blockIdx.x, blockIdx.y, gridDim.y, false);
 }
 
 // The jobs of mxfp8_lora_bwd_batch in one flat grid: job j owns blocks first[j] .. first[j + 1] - 1, `used` row
@@ -646,6 +653,7 @@ struct LoraBwdBatch {
   int64_t ld_q;
   uint8_t* s;
   int64_t s_col_tiles;
+  int tiled;
 };
 
 template <int R, bool kQuant>
@@ -659,7 +667,7 @@ __global__ __launch_bounds__(256, 2) void lora_bwd_batch_kernel(const LoraBwdBat
                                  a.ld_q, a.s, a.s_col_tiles, (int)jb.col_tile_off,
                                  static_cast<const uint16_t*>(jb.xa), jb.ld_xa, static_cast<const uint16_t*>(jb.b),
                                  jb.part_dxa, jb.part_db, static_cast<uint16_t*>(jb.dxa), jb.ld_dxa, jb.scale,
-                                 local % a.used, local / a.used, (int)(jb.N / 128));
+                                 local % a.used, local / a.used, (int)(jb.N / 128), a.tiled != 0);
 }
 
 // 16-byte vectors of fp32 partial sums added in ascending partial order, four loads in flight at a time
@@ -1292,12 +1300,14 @@ extern "C" int mxfp8_lora_bwd(const void* dy, int64_t T, int64_t N, int64_t ld_d
 extern "C" int64_t mxfp8_lora_bwd_batch_chunks(int64_t T, int64_t n_total) { return lora_bwd_rows(T, n_total, 512); }
 
 extern "C" int mxfp8_lora_bwd_batch(const mxfp8_lora_bwd_job* jobs, int64_t n_jobs, int64_t T, int64_t r, void* q,
-                                    int64_t ld_q, void* s, int64_t s_col_tiles, void* stream) {
+                                    int64_t ld_q, void* s, int64_t s_col_tiles, int64_t q_tiled, void* stream) {
   MX_CHECK_ARG(jobs && n_jobs > 0 && n_jobs <= MXFP8_LORA_BWD_MAX_JOBS && T > 0 && (r == 16 || r == 32),
                "mxfp8_lora_bwd_batch: need 1..%d jobs, T > 0, r in {16, 32}", MXFP8_LORA_BWD_MAX_JOBS);
   const bool quant = q != nullptr;
   MX_CHECK_ARG(!quant || (s && ld_q % 16 == 0 && mx_aligned(q, 16) && mx_aligned(s, 4)),
                "mxfp8_lora_bwd_batch: bad code / scale destination");
+  MX_CHECK_ARG(q_tiled == 0 || (q_tiled == 1 && ld_q % 128 == 0),
+               "mxfp8_lora_bwd_batch: q_tiled is 0 or 1, with ld_q the columns of q then");
   int64_t n_total = 0;
   for (int64_t j = 0; j < n_jobs; ++j) {
     const mxfp8_lora_bwd_job& jb = jobs[j];
@@ -1339,6 +1349,7 @@ extern "C" int mxfp8_lora_bwd_batch(const mxfp8_lora_bwd_job* jobs, int64_t n_jo
   a.ld_q = ld_q;
   a.s = (uint8_t*)s;
   a.s_col_tiles = s_col_tiles;
+  a.tiled = (int)q_tiled;
   b.nrs = (int)used;
   b.R = (int)r;
   hipStream_t stm = (hipStream_t)stream;

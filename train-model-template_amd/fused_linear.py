@@ -440,6 +440,32 @@ def _add_dgrad(dx, base, dy, dt):
     return dy @ w if dx is None else dx.addmm_(dy, w)
 
 
+def _st(S, skey, width):
+    """Sᵀ [K, width] (zero columns past S's rows) of the saved S.  This step's form only if the saved S is a view of
+    the same buffer: a backward that runs after the next step's forward has the saved S of its own step (see
+    _PLANS), so it builds Sᵀ from that S."""
+    forms = _CAST.get(skey + ("forms",))
+    if forms is not None and forms.rp == width and _same_buffer(S, forms.S_pad):
+        return forms.St
+    ent = _CAST.get(skey + ("padT", width))
+    if ent is None or ent[0] is not S:
+        pad = torch.cat([S, S.new_zeros(width - S.shape[0], S.shape[1])]) if width > S.shape[0] else S
+        ent = _CAST[skey + ("padT", width)] = (S, pad.t().contiguous())
+    return ent[1]
+
+
+def _tn_job(x2, dS, width, out_dtype):
+    """dA = bf16(dSᵀ·x2) as a job of the token reduction, and its partial-sum scratch.  out_dtype float32 holds the bf16
+    values for fp32 parameters: autograd would cast each bf16 slice to its parameter's dtype anyway (exactly), one
+    kernel per adapter."""
+    import _native
+    T, K = x2.shape
+    out = torch.empty((width, K), dtype=out_dtype, device=x2.device)
+    n_part = _native.lora_tn_chunks(T, K) * width * K
+    part = _native.scratch_f32(n_part, x2.device)[:n_part]  # partial sums, read by the launch's sum kernel
+    return (x2, dS, out, 1.0, False), part
+
+
 def _plain_backward(spec, x2, xS, S, Bs, flat, need_x, dt):
     """Per-layer backward (fused_linear.py:128-196): the base layers' dgrads, then the thin branch as one
     product dS = [s·dy·B of each adapter | dy of each thin linear] against the matching rows of S, and
@@ -538,9 +564,9 @@ def _fused_backward(spec, skey, x2, xS, S, Bs, flat, plan, need_x, dt):
     q = sbuf = None
     tile = 0
     batch = T > 0 and _lora_bwd_batchable(spec, flat, xS)
+    import _native
     if batch:
         # every MX layer's lora_bwd (mxfp8.lora_bwd, lora_bwd_batch) in one call: one launch and one of its sums
-        import _native
         q, sbuf, dbs = _native.host().group_lora_bwd([flat[i] for i in spec.mx], xS, [Bs[sl.index] for sl in batch],
                                                      [sl.col for sl in batch], [sl.scale for sl in batch], dS, need_x,
                                                      _native.stream_of(x2))
@@ -578,43 +604,27 @@ def _fused_backward(spec, skey, x2, xS, S, Bs, flat, plan, need_x, dt):
     a32 = bool(spec.adapters) and all(spec.parts[sl.layer][1].dtype == torch.float32 for sl in spec.adapters)
 
     def tn_job():
-        # bf16(dSᵀ·x2), held in fp32 when every A is an fp32 parameter: autograd would cast each bf16 slice to its
-        # parameter's dtype anyway (exactly), one kernel per adapter.  (job, its partial-sum scratch)
-        import _native
-        out = torch.empty((width, K), dtype=torch.float32 if a32 else dt, device=dev)
-        n_part = _native.lora_tn_chunks(T, K) * width * K
-        part = _native.scratch_f32(n_part, dev)[:n_part]  # partial sums, read by the launch's sum kernel
-        return (x2, dS, out, 1.0, False), part
+        return _tn_job(x2, dS, width, torch.float32 if a32 else dt)
 
     if need_x:
         wq, ws, lay = wt
+        if batch:
+            lay |= _native.GEMM_A_TILED  # group_lora_bwd's codes
         for sl in spec.thin:
             dS[:, sl.cols].copy_(flat[sl.layer])
         codes = (q, sbuf.view(mxfp8.E8))
         if native:
             # bf16(bf16(MX GEMM) + dS·S): the reference's dx.addmm_(dS, S) in the GEMM epilogue
-            # this step's St only if the saved S is a view of the same buffer: a backward that runs after the next
-            # step's forward has the saved S of its own step (see _PLANS), so it builds St from that S
-            forms = _CAST.get(skey + ("forms",))
-            if forms is not None and forms.rp == width and _same_buffer(S, forms.S_pad):
-                St = forms.St
-            else:
-                ent = _CAST.get(skey + ("padT", width))
-                if ent is None or ent[0] is not S:
-                    pad = torch.cat([S, S.new_zeros(width - S.shape[0], S.shape[1])]) if width > S.shape[0] else S
-                    ent = _CAST[skey + ("padT", width)] = (S, pad.t().contiguous())
-                St = ent[1]
-            lora = (dS[:, :r_dx], St[:, :r_dx])
-            import _native
+            lora = (dS[:, :r_dx], _st(S, skey, width)[:, :r_dx])
             if spec.adapters and FOLD_TN[0] and r_dx in (16, 32, 48) and not lay & _native.GEMM_WIDE:
                 # the dA reduction in the dx GEMM's launch: the same bits as the two calls below
                 job, part = tn_job()
                 dA = job[2]
                 dx = mxfp8.mx_mm_tn(*codes, wq, ws, lora, 1.0, lay, T, [job], part)
             else:
-                dx = mxfp8.mx_mm(*codes, wq, ws, layout=lay, lora=lora, alpha=1.0)
+                dx = mxfp8.mx_mm(*codes, wq, ws, layout=lay, lora=lora, alpha=1.0, m=T)
         else:
-            dx = mxfp8.mx_mm(*codes, wq, ws, layout=lay)
+            dx = mxfp8.mx_mm(*codes, wq, ws, layout=lay, m=T)
             for i in spec.plain:  # plain bf16 linears (neither MX nor thin)
                 dx.addmm_(flat[i], spec.parts[i][0].weight.to(dt))
             if dS is not None:
@@ -622,7 +632,6 @@ def _fused_backward(spec, skey, x2, xS, S, Bs, flat, plan, need_x, dt):
         del codes, q, sbuf
     if spec.adapters:
         if native and dA is None:
-            import _native
             job, part = tn_job()
             dA = job[2]
             _native.lora_tn(x2, dS, dA, part)

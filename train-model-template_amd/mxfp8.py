@@ -408,16 +408,24 @@ def _rows_bf16(t):
 
 
 def _quant_act(x):
-    """(codes, scales) of a linear layer's input, reused when x is the live tensor quantized last, at the same
+    """(MX-tiled codes, scales) of a linear layer's input, reused when x is the live tensor quantized last, at the same
     version; STATS counts both cases."""
     codes = _ACT.lookup(x)
     if codes is not None:
         STATS["reuse"] += 1
         return codes
-    codes = mx_quant(_rows_bf16(x))
+    codes = mx_quant_tiled(_rows_bf16(x))
     STATS["quant"] += 1
     _ACT.remember(x, codes)
     return codes
+
+
+def _fwd_operand(lin):
+    """(codes, scales, out, lora, alpha, layout) of mx_mm for a layer's forward from MX-tiled activations: its MX-tiled
+    weight copy where it has one (a gate/up half is a row range of the pair's), else the row-major codes."""
+    pair = lin.__dict__.get("_mx_gu")
+    w = pair[0].w_tl[pair[1] * pair[0].n:(pair[1] + 1) * pair[0].n] if pair is not None else lin.__dict__.get("_mx_w_tl")
+    return (lin._mx_w, lin._mx_ws, None, None, 1.0, 1) if w is None else (w, lin._mx_ws, None, None, 1.0, 3)
 
 
 class _MXLinear(torch.autograd.Function):
@@ -427,14 +435,16 @@ class _MXLinear(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, q, s, lin):
         ctx.lin = lin
-        y = mx_mm(q, s, lin._mx_w, lin._mx_ws)
+        y = mx_mm(q, s, *_fwd_operand(lin), m=x.numel() // x.shape[-1])
         return y.view(x.shape[:-1] + (y.shape[-1],))
 
     @staticmethod
     def backward(ctx, dy):
-        qd, sd = mx_quant(_rows_bf16(dy))
+        d2 = _rows_bf16(dy)
+        qd, sd = mx_quant_tiled(d2)
         STATS["quant"] += 1
-        dx = mx_mm(qd, sd, *mx_wt(ctx.lin))
+        wq, ws, lay = group_operand([ctx.lin])
+        dx = mx_mm(qd, sd, wq, ws, layout=lay | 1, m=d2.shape[0])
         return dx.view(dy.shape[:-1] + (dx.shape[-1],)), None, None, None
 
 
