@@ -334,14 +334,7 @@ std::tuple<OptT, Tensor, Tensor, Tensor, Tensor, Tensor> mlp_backward(
   const mxfp8_lora_tn_job jobs[2] = {{ptr(dy), dy.stride(0), a.at(xsd), R, (float)s_d, 1, fp32_bd, ptr(dBd)},
                                      {ptr(x), x.stride(0), a.at(dxa), 2 * R, 1.f, 0, fp32_a, ptr(dA)}};
   const bool fold = need_x && R == 16;
-  if (!fold && R == 16) {
-    ok(mxfp8_lora_tn_batch(jobs, 2, T, K, chunks, a.f(part), st), "mxfp8_lora_tn_batch");
-  } else if (!fold) {
-    for (int j = 0; j < 2; ++j)
-      ok(mxfp8_lora_tn(jobs[j].x, T, K, jobs[j].ld_x, jobs[j].p, jobs[j].rp, chunks, a.f(part) + (j ? chunks * R * K : 0),
-                       jobs[j].scale, jobs[j].transpose, jobs[j].out_f32, jobs[j].out, st),
-         "mxfp8_lora_tn");
-  }
+  if (!fold) ok(mxfp8_lora_tn_batch(jobs, 2, T, K, chunks, a.f(part), st), "mxfp8_lora_tn_batch");
   if (need_x) {
     const int64_t lay = tt | MXFP8_GEMM_B_PI;
     if (fold)

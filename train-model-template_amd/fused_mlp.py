@@ -373,11 +373,8 @@ class _MLP(torch.autograd.Function):
         dA = torch.empty((2 * R, K), dtype=torch.float32 if fp32_a else dt, device=dy2.device)
         tn_jobs = [(dy2, xsd, dB_d, s_d, True), (x2, dxa, dA, 1.0, False)]
         fold = need_x and 2 * R == 32 and FOLD_TN[0]  # else the reductions run here, before the dx GEMM
-        if not fold and 2 * R <= 32:  # the batch takes ranks 16 and 32
+        if not fold:
             _native.lora_tn_batch(tn_jobs, part)
-        elif not fold:
-            _native.lora_tn(dy2, xsd, dB_d, part[:chunks * R * K], scale=s_d, transpose=True)
-            _native.lora_tn(x2, dxa, dA, part[chunks * R * K:])
         dx = None
         if need_x:
             # dx = bf16(bf16(MX(dg | du) · W_gu) + dxa · S): one K = 2N GEMM with the addmm_ of
