@@ -397,7 +397,8 @@ __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(2, 
     else f.b[k][i - kMB] = frag(st + S::kOffB + k * S::kSliceB, (wn * kNB + i - kMB) * 32 + (lane & 31), c0, sw);
   };
   auto mma = [&](const Frags& f, int x, auto pc) {  // product x of a stage; P: half of the 128-wide K tile (blocks 2P, 2P + 1)
-    const int k = x / (kMB * kNB), i = x / kMB % kNB, j = x % kMB;
+    // serpentine: one operand stays from each product to the next (0.3-0.8% on launches that the power limit bounds)
+    const int k = x / (kMB * kNB), j = x / kNB % kMB, i = (j & 1) ? kNB - 1 - x % kNB : x % kNB;
     const int sa = (int)(f.sa[j] >> sshift), sb = (int)(f.sb[i] >> sshift);
     if ((S::kKS == 2 ? k : decltype(pc)::value) == 0)
       acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.b[k][i], f.a[k][j], acc[i][j], 0, 0, 0, sb, 0, sa);
