@@ -670,29 +670,17 @@ __global__ __launch_bounds__(256, 2) void lora_bwd_batch_kernel(const LoraBwdBat
                                  local % a.used, local / a.used, (int)(jb.N / 128), a.tiled != 0);
 }
 
-// 16-byte vectors of fp32 partial sums added in ascending partial order, four loads in flight at a time
-__device__ __forceinline__ float4 add4(float4 a, float4 b) {
-  return make_float4(a.x + b.x, a.y + b.y, a.z + b.z, a.w + b.w);
-}
 // The partials are read once: streaming (non-temporal) loads.  The backward finish at configuration 3 (graph timing,
 // one box, three alternating pairs, bit-identical): 13.07-13.10 us with plain loads, 12.01-12.03 us with these;
-// lora_bwd's sums unchanged (23.7 / 57.9 us with the main kernel); eight loads in flight instead of four measured
-// the same.  (The forward's sum_parts kernel measured slower with them: 12.8 against 11.6 us.)
+// lora_bwd's sums unchanged (23.7 / 57.9 us with the main kernel).  Six in flight: the finish at T = 1000 / 10752 /
+// 142336 takes 6.2 / 12.3 / 169 us, with eight 5.9 / 12.9 / 172, with four 6.6 / 12.2 / 169.  (The forward's sum_parts kernel measured slower with them: 12.8 against 11.6 us.)
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ float4 ld_part(const float4* p) {
   const f32x4 t = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));
   return make_float4(t.x, t.y, t.z, t.w);
 }
 __device__ __forceinline__ float4 sum_ordered(const float4* __restrict__ p, int64_t stride, int n) {
-  float4 v = ld_part(p);
-  int c = 1;
-  for (; c + 3 < n; c += 4) {
-    const float4 x0 = ld_part(p + c * stride), x1 = ld_part(p + (c + 1) * stride), x2 = ld_part(p + (c + 2) * stride),
-                 x3 = ld_part(p + (c + 3) * stride);
-    v = add4(add4(add4(add4(v, x0), x1), x2), x3);
-  }
-  for (; c < n; ++c) v = add4(v, ld_part(p + c * stride));
-  return v;
+  return ordered_sum<6, float4>(n, [&](int c) { return ld_part(p + c * stride); }, add_to);
 }
 
 // dxa[t, ρ] (row stride ld_dxa) = bf16(scale · Σ_p part_dxa[p, t, ρ]) over the first nx = T·R elements (none when
@@ -767,16 +755,8 @@ __device__ __forceinline__ void tn_sum_body(const float* __restrict__ part, int 
                                             int transpose, int out_f32, void* __restrict__ out, int64_t i) {
   const int64_t n = (int64_t)RP * K;
   if (i >= n) return;
-  float v = part[i];
-  int c = 1;
-  for (; c + 7 < chunks; c += 8) {  // eight loads in flight, added in chunk order
-    float x[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = part[(int64_t)(c + u) * n + i];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) v += x[u];
-  }
-  for (; c < chunks; ++c) v += part[(int64_t)c * n + i];
+  float v = ordered_sum<8, float>(chunks, [&](int c) { return part[(int64_t)c * n + i]; },
+                                  [](float& x, float y) { x += y; });
   v = round_bf16(v);
   if (scale != 1.0f) v = round_bf16(v * scale);
   const int64_t rho = i / K, k = i % K;
@@ -1244,11 +1224,14 @@ extern "C" int mxfp8_res_lora(const void* x, const void* y, const void* xa, int6
 // CU with the LoRA products, whose dB partials grow with the chunk count; three for the codes alone), so the grid
 // runs in one round.  Rounding the chunk count up instead gave dy [10752, 6144] 11 x 48 = 528 workgroups, a second
 // round of 16 for the 512 slots: 58.3 against 52.2 us for 8 x 48 (graph timing, one box).
+// A chunk has at least four 32-row blocks where there are as many, one for each wave: with one or two, the others
+// idled and the sums had two to four times the dB partials (call and sums, us: dy [1500, 1024] 15.3 -> 10.2, [4096,
+// 1024] 16.3 -> 12.3, [1500, 1024 | 256 | 256] 12.8 -> 10.8; [256, *] and longer or wider ones unchanged).
 static int64_t lora_bwd_rows(int64_t T, int64_t N, int64_t target) {
   if (T <= 0 || N <= 0 || N % 128) return 0;
   const int64_t blocks = (T + 127) / 128 * 4;  // 32-row blocks up to the padded end of the last 128-row tile
   const int64_t cs = N / 128, want = std::max<int64_t>(1, target / cs);
-  const int64_t per = (blocks + std::min(want, blocks) - 1) / std::min(want, blocks);
+  const int64_t per = std::max<int64_t>(4, (blocks + std::min(want, blocks) - 1) / std::min(want, blocks));
   return (blocks + per - 1) / per;
 }
 

@@ -530,16 +530,7 @@ __global__ __launch_bounds__(256) void sum_parts_kernel(const float* __restrict_
       a += b;
     }
   };
-  F v = src[0];
-  int64_t p = 1;
-  for (; p + 7 < n_parts; p += 8) {
-    F x[8];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) x[u] = src[(p + u) * stride];
-#pragma unroll
-    for (int u = 0; u < 8; ++u) add(v, x[u]);
-  }
-  for (; p < n_parts; ++p) add(v, src[p * stride]);
+  const F v = ordered_sum<8, F>(n_parts, [&](int64_t p) { return src[p * stride]; }, add);
   const float* f = reinterpret_cast<const float*>(&v);
 #pragma unroll
   for (int k = 0; k < kW; ++k) {

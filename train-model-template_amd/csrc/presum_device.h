@@ -42,21 +42,7 @@ __device__ __forceinline__ void presum_block(const PreSum& a, int b) {
   const int64_t i = (int64_t)b * 256 + threadIdx.x;
   if (i < a.count4) {
     const float4* src = reinterpret_cast<const float4*>(a.part) + i;
-    float4 v = src[0];
-    int p = 1;
-    for (; p + 7 < a.n_parts; p += 8) {
-      float4 x[8];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) x[u] = src[(int64_t)(p + u) * a.count4];
-#pragma unroll
-      for (int u = 0; u < 8; ++u) {
-        v.x += x[u].x; v.y += x[u].y; v.z += x[u].z; v.w += x[u].w;
-      }
-    }
-    for (; p < a.n_parts; ++p) {
-      const float4 x = src[(int64_t)p * a.count4];
-      v.x += x.x; v.y += x.y; v.z += x.z; v.w += x.w;
-    }
+    const float4 v = ordered_sum<8, float4>(a.n_parts, [&](int p) { return src[(int64_t)p * a.count4]; }, add_to);
     const uint32_t lo = f32_to_bf16_bits(v.x * a.scale) | (f32_to_bf16_bits(v.y * a.scale) << 16);
     const uint32_t hi = f32_to_bf16_bits(v.z * a.scale) | (f32_to_bf16_bits(v.w * a.scale) << 16);
     reinterpret_cast<uint2*>(a.out)[i] = make_uint2(lo, hi);
