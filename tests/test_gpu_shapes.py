@@ -1,7 +1,8 @@
 """The workgroup shapes of the MX GEMM (csrc/mx_gemm.hip, pick_shape): 64 x 64, 64 x 128 and 128 x 128 tiles where
-256 x 128 ones would leave CUs idle, 256 x 256 for long launches.  An output element adds the same products over K in
-the same order in every shape, so each size must give the bits of the explicitly asked 8-wave shape run whole
-(MXFP8_GEMM_WIDE without a workspace), which every size takes: bit-exact, no tolerance."""
+256 x 128 ones would leave CUs idle (in a whole launch or in its last rows only), 256 x 256 for long launches.  An
+output element adds the same products over K in the same order in every shape, so each size must give the bits of the
+explicitly asked 8-wave shape run whole (MXFP8_GEMM_WIDE without a workspace), which every size takes: bit-exact, no
+tolerance."""
 import pytest
 import torch
 
@@ -25,7 +26,11 @@ def _operands(M, N, K, gpu):
     (1000, 2048, 1024), (961, 1920, 1408),                                                 # 64 x 128
     (129, 12288, 256), (1500, 2048, 2048), (1921, 1920, 1152),                             # 128 x 128
     (321, 12288, 384), (1025, 12288, 128),                                                 # 256 x 128
-    (5000, 2048, 2048), (4353, 2304, 1280)])                                               # 256 x 256
+    (5000, 2048, 2048), (4353, 2304, 1280),                                                # 256 x 256
+    # 256 x 128, the rows past the last whole round of tiles in 64 x 128 or 128 x 128 tiles: 1 to 704 such rows, after
+    # one workgroup per CU and after two
+    (1281, 12288, 384), (1407, 6144, 256), (3840 + 257, 6272, 640), (8896, 2048, 1152), (5377, 1920, 2048),  # 64 x 128
+    (2753, 12288, 128), (3073, 6272, 640), (9217, 2048, 1152)])                                              # 128 x 128
 @pytest.mark.parametrize("rank", [0, 16, 48])
 def test_every_shape_gives_the_same_bits(M, N, K, rank, gpu):
     g, (qa, sa), (qb, sb), b = _operands(M, N, K, gpu)
@@ -49,7 +54,8 @@ def test_every_shape_gives_the_same_bits(M, N, K, rank, gpu):
     assert torch.equal(ft[0].view(torch.int16), ft[1].view(torch.int16))
 
 
-@pytest.mark.parametrize("M,N,K", [(65, 384, 640), (961, 1920, 1408), (1921, 1920, 1152), (20501, 2048, 12288)])
+@pytest.mark.parametrize("M,N,K", [(65, 384, 640), (961, 1920, 1408), (1921, 1920, 1152), (20501, 2048, 12288),
+                                   (4097, 2048, 1152), (9217, 2048, 1152)])
 def test_folded_launches_in_every_shape(M, N, K, gpu):
     """mxfp8_gemm_nt_sum and mxfp8_gemm_nt_tn against the separate calls, in the shapes that carry the folded work and
     in the 8-wave one, which launches it apart: bit-identical."""

@@ -191,6 +191,7 @@ struct CSeg {
 // Launch plan (computed on the host, see make_plan).
 struct Plan {
   int tm, tn;        // tiles along M and N
+  int m_base;        // first row of the tiles (a multiple of 256)
   int full;          // logical tiles [0, full) run whole
   int per_full;      // full tiles per XCD (ceil(full / 8)); grid part one = 8 * per_full workgroups
   int nsplit;        // logical tiles [full, full + nsplit) split along K
@@ -248,41 +249,22 @@ __device__ __forceinline__ v8i frag(const uint8_t* base, int row, int c0, int sw
   return r;
 }
 
+template <class S>
+constexpr int kRingBytes = S::kStages * S::kStageBytes;
+
+// One tile (or K piece of one) of a launch: workgroup `bid` of the plan's tiles, its ring in `lds`; `arrived` is a
+// workgroup-shared int.
 template <int kR, class S, int kEpi>
-__global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_kernel(
-    const uint8_t* __restrict__ A, const uint8_t* __restrict__ SA, int64_t lda, const uint8_t* __restrict__ B,
-    const uint8_t* __restrict__ SB, int64_t ldb, int M, int N, int K, CSeg cseg, Lora lora, Plan plan, int tiled,
-    SwEpi swe, SwBwd swb, const TnBatch tnb, const PreSum pre) {
+__device__ __forceinline__ void gemm_body(const uint8_t* __restrict__ A, const uint8_t* __restrict__ SA, int64_t lda,
+                                          const uint8_t* __restrict__ B, const uint8_t* __restrict__ SB, int64_t ldb,
+                                          int M, int N, int K, const CSeg& cseg, const Lora& lora, const Plan& plan,
+                                          int tiled, const SwEpi& swe, const SwBwd& swb, const PreSum& pre,
+                                          const int bid, uint8_t* const lds, int& arrived) {
   constexpr int kMB = S::kMB, kNB = S::kNB, kBM = S::kBM;
-  __shared__ __attribute__((aligned(16))) uint8_t lds[S::kStages * S::kStageBytes];
-  __shared__ int arrived;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform (SGPR)
   // compute sub-tile: n rows wn * 32 kNB + [0, 32 kNB), m rows wm * 32 kMB + [0, 32 kMB)
   const int wn = wave / S::kWM, wm = wave % S::kWM;
-
-  // ---- workgroups before the tiles: the sum of the epilogue operand P (mxfp8_gemm_nt_sum, presum_device.h)
-  int bid = blockIdx.x;
-  if constexpr (kFoldSum<kR, S, kEpi>) {
-    if (bid < pre.blocks) {
-      presum_block(pre, bid);
-      return;
-    }
-    bid -= pre.blocks;  // a multiple of 8: the tiles keep their XCDs
-  }
-
-  // ---- workgroups past the tiles: the folded token reductions (mxfp8_gemm_nt_tn), in the ring's LDS.  They are
-  // numbered after every tile, so the dispatcher starts them only once each tile has started, in the slots the
-  // last round of tiles leaves free.
-  if constexpr (kFoldTn<kR, S, kEpi>) {
-    const int first = 8 * (plan.per_full + plan.per_split);
-    if (bid >= first) {
-      uint16_t* tl = reinterpret_cast<uint16_t*>(lds);
-      if (tnb.kd == 2) tn_batch_block<2, true>(tnb, bid - first, tl);
-      else tn_batch_block<1, true>(tnb, bid - first, tl);
-      return;
-    }
-  }
 
   // ---- which tile (and which K piece) this workgroup computes
   const int ns_all = K / kBK;  // even: K % 128 == 0
@@ -304,7 +286,7 @@ __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(2, 
   }
   int mt_, nt_;
   tile_coords<S::kGroupM>(tile, plan.tm, plan.tn, mt_, nt_);
-  const int m0 = mt_ * kBM, n0 = nt_ * S::kBN;
+  const int m0 = plan.m_base + mt_ * kBM, n0 = nt_ * S::kBN;
   const int nkt = K / 128;
 
   // DMA roles: wave w stages A rows w*16*kSA + [0, 16*kSA) and B rows w*16*kSB + [0, 16*kSB) in 1 KB slices
@@ -954,6 +936,50 @@ __global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(2, 
   }
 }
 
+// The launch: summing workgroups (mxfp8_gemm_nt_sum), then the tiles, then the token reductions (mxfp8_gemm_nt_tn).
+// S2: the shape of the rows past the last whole round of S tiles (plan `tail`, pick_shape), or S for none.
+template <int kR, class S, int kEpi, class S2 = S>
+__global__ __launch_bounds__(S::kThreads) __attribute__((amdgpu_waves_per_eu(2, 2))) void gemm_kernel(
+    const uint8_t* __restrict__ A, const uint8_t* __restrict__ SA, int64_t lda, const uint8_t* __restrict__ B,
+    const uint8_t* __restrict__ SB, int64_t ldb, int M, int N, int K, CSeg cseg, Lora lora, Plan plan, int tiled,
+    SwEpi swe, SwBwd swb, const TnBatch tnb, const PreSum pre, const Plan tail) {
+  constexpr bool kTail = !std::is_same_v<S, S2>;
+  static_assert(!kTail || (S::kThreads == S2::kThreads && !std::is_same_v<S, Wide>), "one workgroup size");
+  __shared__ __attribute__((aligned(16))) uint8_t lds[std::max(kRingBytes<S>, kRingBytes<S2>)];
+  __shared__ int arrived;
+  // ---- workgroups before the tiles: the sum of the epilogue operand P (mxfp8_gemm_nt_sum, presum_device.h)
+  int bid = blockIdx.x;
+  if constexpr (kFoldSum<kR, S, kEpi>) {
+    if (bid < pre.blocks) {
+      presum_block(pre, bid);
+      return;
+    }
+    bid -= pre.blocks;  // a multiple of 8: the tiles keep their XCDs
+  }
+  const int tail_first = 8 * (plan.per_full + plan.per_split);  // also a multiple of 8
+
+  // ---- workgroups past the tiles: the folded token reductions (mxfp8_gemm_nt_tn), in the ring's LDS.  They are
+  // numbered after every tile, so the dispatcher starts them only once each tile has started, in the slots the
+  // last round of tiles leaves free.
+  if constexpr (kFoldTn<kR, S, kEpi>) {
+    const int first = tail_first + (kTail ? 8 * tail.per_full : 0);
+    if (bid >= first) {
+      uint16_t* tl = reinterpret_cast<uint16_t*>(lds);
+      if (tnb.kd == 2) tn_batch_block<2, true>(tnb, bid - first, tl);
+      else tn_batch_block<1, true>(tnb, bid - first, tl);
+      return;
+    }
+  }
+  if constexpr (kTail) {
+    if (bid >= tail_first) {
+      gemm_body<kR, S2, kEpi>(A, SA, lda, B, SB, ldb, M, N, K, cseg, lora, tail, tiled, swe, swb, pre,
+                              bid - tail_first, lds, arrived);
+      return;
+    }
+  }
+  gemm_body<kR, S, kEpi>(A, SA, lda, B, SB, ldb, M, N, K, cseg, lora, plan, tiled, swe, swb, pre, bid, lds, arrived);
+}
+
 int cached_cus() {
   static int cus[64] = {0};
   int dev = 0;
@@ -969,10 +995,11 @@ int cached_cus() {
 // Split the tail wave of the Wide shape along K when it would leave more than half of the CUs idle (one workgroup
 // per CU).  Returns the workspace bytes the plan needs (0 without a split).
 template <class S>
-int64_t make_plan(int64_t M, int64_t N, int64_t K, int cus, Plan& p) {
+int64_t make_plan(int64_t M, int64_t N, int64_t K, int cus, Plan& p, int64_t m_base = 0) {
   constexpr bool kSplit = std::is_same_v<S, Wide>;
   const int slots = cus;
-  p.tm = (int)((M + S::kBM - 1) / S::kBM);
+  p.m_base = (int)m_base;
+  p.tm = (int)((M - m_base + S::kBM - 1) / S::kBM);
   p.tn = (int)((N + S::kBN - 1) / S::kBN);
   const int total = p.tm * p.tn, ns = (int)(K / kBK);
   const int rem = total % slots;
@@ -999,17 +1026,17 @@ int64_t make_plan(int64_t M, int64_t N, int64_t K, int cus, Plan& p) {
   return kCounterBytes + (int64_t)p.nsplit * p.parts * S::kPartBytes;
 }
 
-template <class S>
+template <class S, class S2 = S>
 void launch(const uint8_t* A, const uint8_t* SA, int64_t lda, const uint8_t* B, const uint8_t* SB, int64_t ldb,
-            int M, int N, int K, const CSeg& cseg, const Lora& lo, int r, const Plan& plan, int layout,
-            const TnBatch& tnb, int64_t tn_blocks, const PreSum& pre, hipStream_t stm) {
-  dim3 grid((unsigned)(pre.blocks + 8 * plan.per_full + 8 * plan.per_split + tn_blocks));
-#define GEMM_ARGS A, SA, lda, B, SB, ldb, M, N, K, cseg, lo, plan, layout, SwEpi{}, SwBwd{}, tnb, pre
-  if (!lo.p) gemm_kernel<0, S, kEpiPlain><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
-  else if (r == 16) gemm_kernel<16, S, kEpiPlain><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
-  else if (r == 32) gemm_kernel<32, S, kEpiPlain><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
-  else if (r == 48) gemm_kernel<48, S, kEpiPlain><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
-  else gemm_kernel<64, S, kEpiPlain><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
+            int M, int N, int K, const CSeg& cseg, const Lora& lo, int r, const Plan& plan, const Plan& tail,
+            int layout, const TnBatch& tnb, int64_t tn_blocks, const PreSum& pre, hipStream_t stm) {
+  dim3 grid((unsigned)(pre.blocks + 8 * plan.per_full + 8 * plan.per_split + 8 * tail.per_full + tn_blocks));
+#define GEMM_ARGS A, SA, lda, B, SB, ldb, M, N, K, cseg, lo, plan, layout, SwEpi{}, SwBwd{}, tnb, pre, tail
+  if (!lo.p) gemm_kernel<0, S, kEpiPlain, S2><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
+  else if (r == 16) gemm_kernel<16, S, kEpiPlain, S2><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
+  else if (r == 32) gemm_kernel<32, S, kEpiPlain, S2><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
+  else if (r == 48) gemm_kernel<48, S, kEpiPlain, S2><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
+  else gemm_kernel<64, S, kEpiPlain, S2><<<grid, S::kThreads, 0, stm>>>(GEMM_ARGS);
 #undef GEMM_ARGS
 }
 
@@ -1040,23 +1067,49 @@ float shape_us(ShapeId id, int64_t M, int64_t N, int64_t K, int cus) {
 }
 
 // The shape of a plain GEMM (its bits are the same in every shape: an output element's products are added over K in
-// the same order).  us per launch, Tall / the shape taken: M = 256, N = 2048, K = 12288 57 / 23 (Small); M = 1000,
-// N = 2048, K = 6144 32 / 21 (Low); M = 2048, N = 2048, K = 6144 32.2 / 30.7 (Mid); M = 21504, N = 2048, K = 12288
-// 462 / 412 (Wide).  Another shape than Tall has to be 2% faster by the estimate.  wide_ok: N % 256 == 0 and one
-// output; wide_more: us that the launches which Wide cannot fold into its own cost.
-ShapeId pick_shape(int64_t M, int64_t N, int64_t K, int cus, bool wide_ok, float wide_more) {
-  ShapeId best = ShapeId::kTall;
-  float t = shape_us(best, M, N, K, cus) * 0.98f;
+// the same order), and of its tail: the rows of a Tall launch from tail_row on, in smaller tiles of the same launch.
+struct Pick {
+  ShapeId shape;
+  ShapeId tail;      // kMid or kLow, with
+  int64_t tail_row;  // the first of its rows, a multiple of 256; 0: no tail
+};
+
+// us per launch, Tall / the shape taken: M = 256, N = 2048, K = 12288 57 / 23 (Small); M = 1000, N = 2048, K = 6144
+// 32 / 21 (Low); M = 2048, N = 2048, K = 6144 32.2 / 30.7 (Mid); M = 21504, N = 2048, K = 12288 462 / 412 (Wide).
+// A tail starts after the last whole round of one or two Tall workgroups per CU, where a few more 256 x 128 tiles
+// would run alone, a CU each (0.30 us a K step against Low's 0.15): M = 8896, N = 2048, K = 12288 203 / 177 (48 tiles
+// past 512, in Low); M = 9254, N = 2048, K = 6144 121 / 111 (Mid); M = 17960, N = 1024, K = 7168 123 / 108 (Low).
+// M = 10752, N = 2048 leaves 160 tiles past 512 and stays whole, 240 / 257.  Over 85 sizes of 300 to 1700 tiles the
+// tails take 2.5% off on average and no size got slower.  Another shape or a tail has to be 2% faster than Tall by
+// the estimate.  wide_ok: N % 256 == 0 and one output; wide_more: us that the launches which Wide cannot fold into
+// its own cost.
+Pick pick_shape(int64_t M, int64_t N, int64_t K, int cus, bool wide_ok, float wide_more) {
+  Pick best{ShapeId::kTall, ShapeId::kTall, 0};
+  float t = shape_us(best.shape, M, N, K, cus) * 0.98f;
   for (ShapeId id : {ShapeId::kWide, ShapeId::kMid, ShapeId::kLow, ShapeId::kSmall}) {
     if (id == ShapeId::kWide && !(wide_ok && N % 256 == 0)) continue;
     const float e = shape_us(id, M, N, K, cus) + (id == ShapeId::kWide ? wide_more : 0.f);
     if (e < t) {
-      best = id;
+      best.shape = id;
       t = e;
+    }
+  }
+  const int64_t tn = (N + 127) / 128, tm = (M + 255) / 256;
+  for (int64_t per : {(int64_t)2 * cus, (int64_t)cus}) {
+    const int64_t head = tm * tn / per * per / tn;  // rows of tiles in whole rounds
+    if (head < 1 || head >= tm) continue;
+    for (ShapeId id : {ShapeId::kMid, ShapeId::kLow}) {
+      const float e = shape_us(ShapeId::kTall, head * 256, N, K, cus) + shape_us(id, M - head * 256, N, K, cus) -
+                      kCost[(int)id].base;
+      if (e < t) {
+        best = Pick{ShapeId::kTall, id, head * 256};
+        t = e;
+      }
     }
   }
   return best;
 }
+
 // us of a token reduction or a partial sum in a launch of its own beyond its share of a folded launch (measured at
 // T = 10752: dx with its reductions 252 folded, 237 + 29 apart; down with its sum 135 against 124 + 13).
 constexpr float kUnfoldedTn = 12.f, kUnfoldedSum = 2.f;
@@ -1074,7 +1127,8 @@ namespace {
 int gemm_impl(const void* a, const void* sa, int64_t lda, const void* b, const void* sb, int64_t ldb, int64_t M,
               int64_t N, int64_t K, CSeg cseg, const void* lora_p, int64_t ld_p, const void* lora_q, int64_t ld_q,
               int64_t r, float alpha, int64_t layout, void* workspace, int64_t workspace_bytes, void* stream,
-              const TnBatch& tnb = TnBatch{}, int64_t tn_blocks = 0, const PreSum& pre = PreSum{}, int shape_id = -1) {
+              const TnBatch& tnb = TnBatch{}, int64_t tn_blocks = 0, const PreSum& pre = PreSum{},
+              const Pick* picked = nullptr) {
   void* const c = cseg.ptr[0];
   int64_t ldc = cseg.ld[0];
   MX_CHECK_ARG(a && sa && b && sb && c, "mxfp8_gemm_nt: null pointer");
@@ -1111,16 +1165,21 @@ int gemm_impl(const void* a, const void* sa, int64_t lda, const void* b, const v
   Plan plan;
   const int cus = cached_cus();
   const bool wide = layout & MXFP8_GEMM_WIDE;
-  const ShapeId shape = wide            ? ShapeId::kWide
-                        : shape_id >= 0 ? (ShapeId)shape_id
-                                        : pick_shape(M, N, K, cus, cseg.n == 1, 0.f);
+  const Pick pick = wide     ? Pick{ShapeId::kWide, ShapeId::kWide, 0}
+                    : picked ? *picked
+                             : pick_shape(M, N, K, cus, cseg.n == 1, 0.f);
   int64_t need = 0;
-  switch (shape) {
-    case ShapeId::kTall: need = make_plan<Tall>(M, N, K, cus, plan); break;
+  Plan tail{};
+  switch (pick.shape) {
+    case ShapeId::kTall: make_plan<Tall>(pick.tail_row ? pick.tail_row : M, N, K, cus, plan); break;
     case ShapeId::kWide: need = make_plan<Wide>(M, N, K, cus, plan); break;
     case ShapeId::kMid: need = make_plan<Mid>(M, N, K, cus, plan); break;
     case ShapeId::kLow: need = make_plan<Low>(M, N, K, cus, plan); break;
     case ShapeId::kSmall: need = make_plan<Small>(M, N, K, cus, plan); break;
+  }
+  if (pick.tail_row) {
+    if (pick.tail == ShapeId::kMid) make_plan<Mid>(M, N, K, cus, tail, pick.tail_row);
+    else make_plan<Low>(M, N, K, cus, tail, pick.tail_row);
   }
   if (need > workspace_bytes || (need && !wide)) {  // no (or too small a) workspace: run every tile whole
     plan.full = plan.tm * plan.tn;
@@ -1135,10 +1194,15 @@ int gemm_impl(const void* a, const void* sa, int64_t lda, const void* b, const v
   const uint8_t *A = (const uint8_t*)a, *SA = (const uint8_t*)sa, *B = (const uint8_t*)b, *SB = (const uint8_t*)sb;
   const int tiled = (int)(layout & ~MXFP8_GEMM_WIDE);
   hipStream_t stm = (hipStream_t)stream;
-#define GEMM_LAUNCH(S) \
-  launch<S>(A, SA, lda, B, SB, ldb, (int)M, (int)N, (int)K, cseg, lo, (int)r, plan, tiled, tnb, tn_blocks, pre, stm)
-  switch (shape) {
-    case ShapeId::kTall: GEMM_LAUNCH(Tall); break;
+#define GEMM_LAUNCH(...)                                                                                              \
+  launch<__VA_ARGS__>(A, SA, lda, B, SB, ldb, (int)M, (int)N, (int)K, cseg, lo, (int)r, plan, tail, tiled, tnb,       \
+                      tn_blocks, pre, stm)
+  switch (pick.shape) {
+    case ShapeId::kTall:
+      if (!pick.tail_row) GEMM_LAUNCH(Tall);
+      else if (pick.tail == ShapeId::kMid) GEMM_LAUNCH(Tall, Mid);
+      else GEMM_LAUNCH(Tall, Low);
+      break;
     case ShapeId::kWide: GEMM_LAUNCH(Wide); break;
     case ShapeId::kMid: GEMM_LAUNCH(Mid); break;
     case ShapeId::kLow: GEMM_LAUNCH(Low); break;
@@ -1183,10 +1247,10 @@ extern "C" int mxfp8_gemm_nt_tn(const void* a, const void* sa, int64_t lda, cons
   cs.ptr[0] = (uint16_t*)c;
   cs.ld[0] = ldc;
   // the 8-wave shape does not carry the reductions: they get their own launch
-  const ShapeId shape = N > 0 && K > 0 ? pick_shape(M, N, K, cached_cus(), true, kUnfoldedTn) : ShapeId::kTall;
-  const bool fold = shape != ShapeId::kWide;
+  const Pick pick = N > 0 && K > 0 ? pick_shape(M, N, K, cached_cus(), true, kUnfoldedTn) : Pick{};
+  const bool fold = pick.shape != ShapeId::kWide;
   rc = gemm_impl(a, sa, lda, b, sb, ldb, M, N, K, cs, lora_p, ld_p, lora_q, ld_q, r, alpha, layout, nullptr, 0, stream,
-                 tnb, fold ? nb : 0, PreSum{}, (int)shape);
+                 tnb, fold ? nb : 0, PreSum{}, &pick);
   if (rc == MXFP8_OK && !fold) rc = tn_batch_launch(tnb, nb, (hipStream_t)stream, "mxfp8_gemm_nt_tn");
   if (rc != MXFP8_OK) return rc;
   return tn_sum_batch_launch(sa_tn, ns, (hipStream_t)stream, "mxfp8_gemm_nt_tn");
@@ -1254,13 +1318,13 @@ extern "C" int mxfp8_gemm_nt_sum(const void* a, const void* sa, int64_t lda, con
   // bits, before the plain GEMM.
   // The 8-wave shape has no summing workgroups either.
   hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
-  const ShapeId shape = N > 0 && K > 0 ? pick_shape(M, N, K, cached_cus(), true, kUnfoldedSum) : ShapeId::kTall;
-  if (shape == ShapeId::kWide || hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess ||
+  const Pick pick = N > 0 && K > 0 ? pick_shape(M, N, K, cached_cus(), true, kUnfoldedSum) : Pick{};
+  if (pick.shape == ShapeId::kWide || hipStreamIsCapturing((hipStream_t)stream, &cap) != hipSuccess ||
       cap != hipStreamCaptureStatusNone) {
     const int rc = mxfp8_sum_parts(part, n_parts, M * r, part_scale, lora_p, 1, stream);
     if (rc != MXFP8_OK) return rc;
     return gemm_impl(a, sa, lda, b, sb, ldb, M, N, K, cs, lora_p, r, lora_q, ld_q, r, alpha, layout, nullptr, 0,
-                     stream, TnBatch{}, 0, PreSum{}, (int)shape);
+                     stream, TnBatch{}, 0, PreSum{}, &pick);
   }
   unsigned long long* flags = presum_flags_on_current_device();
   if (!flags) return MXFP8_ERR_ARG;
@@ -1278,7 +1342,7 @@ extern "C" int mxfp8_gemm_nt_sum(const void* a, const void* sa, int64_t lda, con
   pre.wait_limit = wait_limit < 0 ? (1 << 20) : (int)std::min<int64_t>(wait_limit, 1 << 30);
   pre.scale = part_scale;
   return gemm_impl(a, sa, lda, b, sb, ldb, M, N, K, cs, lora_p, r, lora_q, ld_q, r, alpha, layout, nullptr, 0, stream,
-                   TnBatch{}, 0, pre, (int)shape);
+                   TnBatch{}, 0, pre, &pick);
 }
 
 extern "C" int mxfp8_gemm_nt_seg(const void* a, const void* sa, int64_t lda, const void* b, const void* sb,
@@ -1344,7 +1408,7 @@ extern "C" int mxfp8_gemm_swiglu_fwd(const void* a, const void* sa, const void* 
   const uint8_t *A = (const uint8_t*)a, *SA = (const uint8_t*)sa, *B = (const uint8_t*)b, *SB = (const uint8_t*)sb;
 #define SWIGLU_LAUNCH(R, S)                                                                                        \
   gemm_kernel<R, S, kEpiSwiGluFwd><<<grid, S::kThreads, 0, stm>>>(A, SA, K, B, SB, K, (int)M, (int)(2 * N), (int)K, cs, \
-                                                                  Lora{}, plan, tiled, sw, SwBwd{}, TnBatch{}, PreSum{})
+                                                                  Lora{}, plan, tiled, sw, SwBwd{}, TnBatch{}, PreSum{}, Plan{})
   if (mid) {
     if (r == 16) SWIGLU_LAUNCH(16, Mid);
     else SWIGLU_LAUNCH(32, Mid);
@@ -1390,7 +1454,7 @@ extern "C" int mxfp8_gemm_swiglu_bwd(const void* a, const void* sa, const void* 
   const int tiled = MXFP8_GEMM_A_TILED | MXFP8_GEMM_B_TILED;
   gemm_kernel<16, Tall, kEpiSwiGluBwd><<<grid, Tall::kThreads, 0, (hipStream_t)stream>>>(
       (const uint8_t*)a, (const uint8_t*)sa, K, (const uint8_t*)b, (const uint8_t*)sb, K, (int)M, (int)N, (int)K, cs,
-      Lora{}, plan, tiled, SwEpi{}, sw, TnBatch{}, PreSum{});
+      Lora{}, plan, tiled, SwEpi{}, sw, TnBatch{}, PreSum{}, Plan{});
   MX_CHECK_LAUNCH("mxfp8_gemm_swiglu_bwd");
   return MXFP8_OK;
 }
