@@ -186,16 +186,17 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFwdWavesPe
 //     then h rows to its LDS tile and reads each back column-wise with ds_read_b64_tr_b16; accumulated over
 //     the super-block in registers and stored after it.
 // The large operands of the next row block (gu, dhm) are loaded one row block ahead.  The small per-row operands
-// (xs, dxd and their transposed copies, L2-resident; the same 6 KB at r = 16 for every wave of the workgroup):
-//   r = 16 (kStage): staged in LDS one row block ahead, by global_load_lds DMAs issued at the start of the row
+// (xs, dxd and their transposed copies, L2-resident; the same 6 r / 16 KB for every wave of the workgroup):
+//   r = 16, and r = 32 with 8 waves (kStage): staged in LDS one row block ahead, by global_load_lds DMAs issued at the start of the row
 //     block before (each 1 KB DMA lands as the lane-ordered MFMA operand, so the reads are conflict-free
 //     ds_read_b128), one copy per workgroup instead of one per wave.  Each wave drains its memory counter before
 //     the row block's barrier, and the block's code, scale and partial stores are issued after that barrier:
 //     the memory counter completes in issue order, so a wait for a load issued behind a store also waits for
 //     the store, and the previous form's first wait of every row block (for the small loads, issued behind the
 //     previous block's stores) paid the stores' latency.  Configuration 3, graph timing, two alternating pairs
-//     on one box, outputs bit-identical: 148.1-149.6 against 140.8-144.4 us;
-//   r = 32: loaded per wave at the start of each row block, before the next block's large operands, so
+//     on one box, outputs bit-identical: 148.1-149.6 against 140.8-144.4 us; r = 32, 8 waves (12 KB a row block for
+//     each of the 8 waves, through L1), N = 6144, us: T = 1000 47.8 -> 38.0, T = 2048 78 -> 56, T = 10752 297 -> 204;
+//   r = 32 with 4 waves: loaded per wave at the start of each row block, before the next block's large operands, so
 //     waiting for them leaves the prefetch in flight (the staged form's 24 KB would lower the 4-wave kernel's
 //     workgroups per CU).
 // Rows past T quantize row T - 1 again (the same bytes) and then zero their values, so they add nothing to
@@ -226,7 +227,7 @@ __global__ __launch_bounds__(256 * kQ) __attribute__((amdgpu_waves_per_eu(2, 8))
   // kRB buffers of the per-wave products: with two, row block b fills buffer b % 2 while the waves still sum
   // block b - 1's, so one barrier per row block suffices; taken where they fit the LDS of the workgroups a CU
   // holds now (one with 8 waves, two with 4)
-  constexpr bool kStage = R == 16;                                      // small operands staged in LDS
+  constexpr bool kStage = R == 16 || kQ == 2;                           // small operands staged in LDS
   constexpr int kOps = 6 * (R / 16), kOpDma = (kOps + kW - 1) / kW;  // 1 KB operand images, DMAs per wave
   constexpr int kRedBytes = kW * 32 * (3 * R + 1) * 4, kTrBytes = kW * 32 * kTrLd * 2;
   constexpr int kStageBytes = kStage ? 2 * kOps * 1024 : 0, kLdsCap = (kQ == 2 ? 160 : 80) * 1024;
