@@ -391,8 +391,7 @@ __global__ __launch_bounds__(256 * kQ) __attribute__((amdgpu_waves_per_eu(2, 8))
       uint4 cg = {}, cu = {};
       uint32_t eg = 0, eu = 0;
       if (kQuant) {
-        eg = quant16_codes(dgw, cg);
-        eu = quant16_codes(duw, cu);
+        quant16_codes(dgw, duw, cg, cu, eg, eu);
         if (!kStage) {
           quant16_store(cg, eg, m, live, q, mc, 2 * N, q_tiled, jb + lg * 16, s, 2 * N / 128);
           quant16_store(cu, eu, m, live, q, mc, 2 * N, q_tiled, N + jb + lg * 16, s, 2 * N / 128);

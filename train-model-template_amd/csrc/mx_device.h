@@ -114,22 +114,34 @@ __device__ __forceinline__ u16x2 absmax2(u16x2 acc, uint32_t w) {
 // fp32 bit pattern of the larger half (the block amax as fp32 bits)
 __device__ __forceinline__ uint32_t amax_bits(u16x2 m) { return (uint32_t)max(m.x, m.y) << 16; }
 
-// Four bf16 (two packed words) of a block with scale byte e -> four E4M3 codes.  Finite blocks (e <= 253)
-// use v_cvt_scalef32_pk_fp8_bf16, which computes RNE_E4M3(x / scale) (verified bit-exact on the device for
+// kN times four bf16 (words 2k, 2k + 1 of w) of blocks with scale bytes e(k) -> four E4M3 codes each.  Finite blocks
+// (e <= 253) use v_cvt_scalef32_pk_fp8_bf16, which computes RNE_E4M3(x / scale) (verified bit-exact on the device for
 // every finite bf16 input and power-of-two scale); x / 2^(e-127) = x * 2^(127-e) exactly, and e == 0 scales
 // by 1.  RCEIL guarantees |x| / scale <= 448 there, so no clamp is needed.  Blocks with NaN (e = 255) or inf
 // (e = 254) take encode4, which clamps inf to +-448 and writes 0x7F for NaN blocks; the choice is made per
-// wave (ballot) so the common path stays branch- and select-free.
-__device__ __forceinline__ uint32_t encode4_bf16(uint32_t w0, uint32_t w1, uint32_t e) {
-  const float sc = __uint_as_float(e == 0u ? 0x3f800000u : e << 23);
-  s16x2 r = {0, 0};
-  r = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(r, __builtin_bit_cast(bf16x2, w0), sc, false);
-  r = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(r, __builtin_bit_cast(bf16x2, w1), sc, true);
-  uint32_t c = __builtin_bit_cast(uint32_t, r);
-  if (__builtin_amdgcn_ballot_w64(e >= 254u)) {
-    if (e >= 254u) c = encode4(bf16_lo(w0), bf16_hi(w0), bf16_lo(w1), bf16_hi(w1), e);
+// wave (ballot) and once for all kN words, so the common path stays branch- and select-free and the code around it
+// one block for the scheduler (a branch per word took the fused MLP backward at r = 32, N = 6144, T = 10752 204 us,
+// one per row block's 8 words 195; r = 16 146 -> 143).
+template <int kN, class E>
+__device__ __forceinline__ void encode_bf16(const uint32_t* w, E&& e, uint32_t* c) {
+  uint32_t top = 0;
+#pragma unroll
+  for (int k = 0; k < kN; ++k) {
+    const float sc = __uint_as_float(e(k) == 0u ? 0x3f800000u : e(k) << 23);
+    s16x2 r = {0, 0};
+    r = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(r, __builtin_bit_cast(bf16x2, w[2 * k]), sc, false);
+    r = __builtin_amdgcn_cvt_scalef32_pk_fp8_bf16(r, __builtin_bit_cast(bf16x2, w[2 * k + 1]), sc, true);
+    c[k] = __builtin_bit_cast(uint32_t, r);
+    top = max(top, e(k));
   }
-  return c;
+  if (__builtin_expect(__builtin_amdgcn_ballot_w64(top >= 254u) != 0, 0)) {
+#pragma unroll
+    for (int k = 0; k < kN; ++k) {
+      const uint32_t w0 = w[2 * k], w1 = w[2 * k + 1];
+      const uint32_t s = encode4(bf16_lo(w0), bf16_hi(w0), bf16_lo(w1), bf16_hi(w1), e(k));
+      c[k] = e(k) >= 254u ? s : c[k];
+    }
+  }
 }
 
 // The pair {v[l], v[l ^ 32]} (pair32) or {v[l], v[l ^ 16]} (pair16) in every lane l, in either order, from one
@@ -236,16 +248,36 @@ __device__ __forceinline__ void store_scale(uint8_t* p, uint8_t e) {
 }
 
 // The 16 codes of w (with the partner lane's 16 forming the 32-block) into c; returns the block's E8M0 scale.
-__device__ __forceinline__ uint32_t quant16_codes(const uint32_t* w, uint4& c) {
+__device__ __forceinline__ uint32_t quant16_scale(const uint32_t* w) {
   u16x2 mm = {0, 0};
 #pragma unroll
   for (int k = 0; k < 8; ++k) mm = absmax2(mm, w[k]);
   uint32_t a, b;
   pair32(amax_bits(mm), a, b);  // the partner lane l ^ 32 holds the block's other 16 values
-  const uint32_t e = e8m0_from_amax_bits(max(a, b));
-  c = make_uint4(encode4_bf16(w[0], w[1], e), encode4_bf16(w[2], w[3], e), encode4_bf16(w[4], w[5], e),
-                 encode4_bf16(w[6], w[7], e));
+  return e8m0_from_amax_bits(max(a, b));
+}
+__device__ __forceinline__ uint32_t quant16_codes(const uint32_t* w, uint4& c) {
+  const uint32_t e = quant16_scale(w);
+  uint32_t cw[4];
+  encode_bf16<4>(w, [&](int) { return e; }, cw);
+  c = make_uint4(cw[0], cw[1], cw[2], cw[3]);
   return e;
+}
+// Two blocks' (w0, w1) at once, with one branch
+__device__ __forceinline__ void quant16_codes(const uint32_t* w0, const uint32_t* w1, uint4& c0, uint4& c1, uint32_t& e0,
+                                              uint32_t& e1) {
+  const uint32_t a = quant16_scale(w0), b = quant16_scale(w1);
+  uint32_t w[16], cw[8];
+#pragma unroll
+  for (int i = 0; i < 8; ++i) {
+    w[i] = w0[i];
+    w[8 + i] = w1[i];
+  }
+  encode_bf16<8>(w, [&](int k) { return k < 4 ? a : b; }, cw);
+  c0 = make_uint4(cw[0], cw[1], cw[2], cw[3]);
+  c1 = make_uint4(cw[4], cw[5], cw[6], cw[7]);
+  e0 = a;
+  e1 = b;
 }
 
 // The stores of quant16: codes c of row mc, scale byte e of row m (0 for padded rows)

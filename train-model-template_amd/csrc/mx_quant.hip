@@ -39,7 +39,10 @@ __device__ __forceinline__ uint2 quant8(uint4 v, uint32_t& e_out) {
   const uint32_t am = quad_umax(amax_bits(m));
   const uint32_t e = e8m0_from_amax_bits(am);
   e_out = e;
-  return make_uint2(encode4_bf16(v.x, v.y, e), encode4_bf16(v.z, v.w, e));
+  const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+  uint32_t c[2];
+  encode_bf16<2>(w, [&](int) { return e; }, c);
+  return make_uint2(c[0], c[1]);
 }
 
 // The low (or high) bf16 halves of a and b as one packed pair, a's in the low half.
@@ -111,10 +114,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(6, 8))
       // codes of xᵀ rows c, c + 1 (tile-local), columns rl0..rl0+7: one 8-byte slot of each LDS row, slot
       // rl0 / 8 = 4w + rg XOR-swizzled by (c / 8) & 14, which spreads a write instruction over all 64 banks
       // and keeps the slot pairs of a 16-byte read-back together
-      const uint2 c0 = make_uint2(encode4_bf16(pack_lo(w0, w1), pack_lo(w2, w3), e0),
-                                  encode4_bf16(pack_lo(w4, w5), pack_lo(w6, w7), e0));
-      const uint2 c1 = make_uint2(encode4_bf16(pack_hi(w0, w1), pack_hi(w2, w3), e1),
-                                  encode4_bf16(pack_hi(w4, w5), pack_hi(w6, w7), e1));
+      const uint32_t cols[8] = {pack_lo(w0, w1), pack_lo(w2, w3), pack_lo(w4, w5), pack_lo(w6, w7),
+                                pack_hi(w0, w1), pack_hi(w2, w3), pack_hi(w4, w5), pack_hi(w6, w7)};
+      uint32_t cc[4];
+      encode_bf16<4>(cols, [&](int k) { return k < 2 ? e0 : e1; }, cc);
+      const uint2 c0 = make_uint2(cc[0], cc[1]), c1 = make_uint2(cc[2], cc[3]);
       const int c = ch * 8 + 2 * p;
       const int slot = (4 * w + rg) ^ (ch & 14);
       *reinterpret_cast<uint2*>(qtt + c * kLdC + slot * 8) = c0;
