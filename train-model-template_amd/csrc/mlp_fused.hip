@@ -208,13 +208,19 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFwdWavesPe
 // bytes written here and read by the finish); one workgroup per CU (116 KB of LDS at r = 16), still two waves
 // per SIMD.  With two product buffers (r = 16) one barrier per row block replaces two: 1-4% faster alone
 // (151.9-154.7 against 148.9-152.4 us at configuration 3, three alternating pairs on one box, bit-identical).
+// The products are written, summed and stored in 16-byte pieces (rows of 3r + 4 floats: the 16 lanes that an LDS access
+// serves at a time start in different banks); kMain fixes the FT and MX-tiled layouts, the ones of the fused path, at
+// compile time (with r = 32 it spills more and was slower).  A row block is bound by its serial chain (VALU about 60%
+// of it, its barrier, these LDS passes), not by memory: us with 4-byte pieces -> 16-byte pieces -> kMain, r = 16,
+// N = 6144: T = 2048 36.8 -> 35.7 -> 35.2, T = 10752 144 -> 138 -> 136; r = 32, T = 10752 195 -> 183.
 // gu is read once here, with non-temporal loads, so it does not push dhm (written by the GEMM just before) and
 // the MX(dg | du) codes out of the last-level cache (with the gate|up epilogue's non-temporal gu stores, MX_NT_GU
 // in mx_gemm.hip: 10-17 us per configuration-3 step faster over five A/B pairs on one box).
 #ifndef MX_BWD_NT_LOAD
 #define MX_BWD_NT_LOAD 1
 #endif
-template <int R, bool kQuant, bool kDgu, int kQ = 1>
+typedef float v4f_u __attribute__((ext_vector_type(4), aligned(4)));  // dxa_part is only known to be 4-byte aligned
+template <int R, bool kQuant, bool kDgu, int kQ = 1, bool kMain = false>
 __global__ __launch_bounds__(256 * kQ) __attribute__((amdgpu_waves_per_eu(2, 8))) void bwd_kernel(
     const uint16_t* __restrict__ gu, const uint16_t* __restrict__ xs, const uint16_t* __restrict__ xsT,
     const uint16_t* __restrict__ dhm, const uint16_t* __restrict__ dxd, const uint16_t* __restrict__ dxdT,
@@ -223,17 +229,18 @@ __global__ __launch_bounds__(256 * kQ) __attribute__((amdgpu_waves_per_eu(2, 8))
     int Tpad, int N, int SB, int CG, float s_g, float s_u, uint8_t* __restrict__ q, uint8_t* __restrict__ s,
     float* __restrict__ dxa_part, float* __restrict__ dbg_part, float* __restrict__ dbu_part,
     float* __restrict__ dad_part, uint16_t* __restrict__ dgu_out, bool q_tiled, bool gu_ft) {
+  if constexpr (kMain) q_tiled = gu_ft = true;
   constexpr int kW = 4 * kQ, kCols = 128 * kQ;  // waves, columns per pass over the column group
   // kRB buffers of the per-wave products: with two, row block b fills buffer b % 2 while the waves still sum
   // block b - 1's, so one barrier per row block suffices; taken where they fit the LDS of the workgroups a CU
   // holds now (one with 8 waves, two with 4)
   constexpr bool kStage = R == 16 || kQ == 2;                           // small operands staged in LDS
   constexpr int kOps = 6 * (R / 16), kOpDma = (kOps + kW - 1) / kW;  // 1 KB operand images, DMAs per wave
-  constexpr int kRedBytes = kW * 32 * (3 * R + 1) * 4, kTrBytes = kW * 32 * kTrLd * 2;
+  constexpr int kRedLd = 3 * R + 4, kRedBytes = kW * 32 * kRedLd * 4, kTrBytes = kW * 32 * kTrLd * 2;
   constexpr int kStageBytes = kStage ? 2 * kOps * 1024 : 0, kLdsCap = (kQ == 2 ? 160 : 80) * 1024;
   constexpr int kRB = 2 * kRedBytes + kTrBytes + kStageBytes <= kLdsCap ? 2 : 1;
   static_assert(kRB * kRedBytes + kTrBytes + kStageBytes <= kLdsCap, "LDS of the workgroups a CU holds");
-  __shared__ float red[kRB][kW][32][3 * R + 1];                        // per-wave dxa | dxa_u | xS products
+  __shared__ __attribute__((aligned(16))) float red[kRB][kW][32][kRedLd];  // per-wave dxa | dxa_u | xS products
   __shared__ __attribute__((aligned(16))) uint16_t trt[kW][32 * kTrLd];  // per-wave dg, then du, then h rows
   // two row blocks' small operands: images xg, xu, xd, tg, tu, td (R / 16 each), lane l's 16 bytes at 16 l
   __shared__ __attribute__((aligned(16))) uint8_t sop[kStage ? 2 : 1][kStage ? kOps : 1][kStage ? 1024 : 16];
@@ -401,33 +408,27 @@ __global__ __launch_bounds__(256 * kQ) __attribute__((amdgpu_waves_per_eu(2, 8))
 #pragma unroll
         for (int i = 0; i < 8; ++i) dgw[i] = duw[i] = hw[i] = 0u;
       }
+      auto red_store = [&](const v16f& p, int col) {  // four adjacent ρ in a register quad: 16-byte stores
+#pragma unroll
+        for (int g = 0; g < R / 8; ++g)
+          *reinterpret_cast<float4*>(&red[buf][w][lane & 31][col + g * 8 + lg * 4]) =
+              make_float4(p[4 * g], p[4 * g + 1], p[4 * g + 2], p[4 * g + 3]);
+      };
       // dxa_g | dxa_u | xS_down products over this tile's columns, D[ρ][m] -> LDS (lane l: m = l % 32,
       // ρ = tile_col(i, l))
       {
         v16f p = v16f{};
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fbg[ks], words_bf8(dgw + 4 * ks), p, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int rr = tile_col(i, lane);
-          if (rr < R) red[buf][w][lane & 31][rr] = p[i];
-        }
+        red_store(p, 0);
         p = v16f{};
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fbu[ks], words_bf8(duw + 4 * ks), p, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int rr = tile_col(i, lane);
-          if (rr < R) red[buf][w][lane & 31][R + rr] = p[i];
-        }
+        red_store(p, R);
         p = v16f{};
 #pragma unroll
         for (int ks = 0; ks < 2; ++ks) p = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fad[ks], words_bf8(hw + 4 * ks), p, 0, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 16; ++i) {
-          const int rr = tile_col(i, lane);
-          if (rr < R) red[buf][w][lane & 31][2 * R + rr] = p[i];
-        }
+        red_store(p, 2 * R);
       }
       // dB_g, dB_u, dA_dᵀ: D[j][ρ] += Σ_m dg[m, j] xs_g[m, ρ] etc. over the 32 rows (one k = 32 step)
       // one transpose tile per wave, refilled three times: a wave's LDS operations run in order, so each store
@@ -464,12 +465,17 @@ __global__ __launch_bounds__(256 * kQ) __attribute__((amdgpu_waves_per_eu(2, 8))
         quant16_store(cu, eu, m, live, q, mc, 2 * N, q_tiled, N + jb + lg * 16, s, 2 * N / 128);
       }
       float* qpart = dxa_part + ((int64_t)(blockIdx.y * (CG / kCols) + oc) * T + rb) * 3 * R;
-      for (int idx = threadIdx.x; idx < 32 * 3 * R; idx += 256 * kQ) {
-        const int mm = idx / (3 * R), cc = idx % (3 * R);
-        float v = red[buf][0][mm][cc];
+      constexpr int kQuads = 32 * 3 * R / 4;
 #pragma unroll
-        for (int u = 1; u < kW; ++u) v += red[buf][u][mm][cc];
-        if (rb + mm < T) qpart[idx] = v;
+      for (int i0 = 0; i0 < kQuads; i0 += 256 * kQ) {
+        const int idx = i0 + threadIdx.x;
+        if (kQuads % (256 * kQ) == 0 || idx < kQuads) {
+          const int mm = idx / (3 * R / 4), cc = 4 * (idx % (3 * R / 4));
+          float4 v = *reinterpret_cast<const float4*>(&red[buf][0][mm][cc]);
+#pragma unroll
+          for (int u = 1; u < kW; ++u) add_to(v, *reinterpret_cast<const float4*>(&red[buf][u][mm][cc]));
+          if (rb + mm < T) *reinterpret_cast<v4f_u*>(qpart + 4 * idx) = v4f_u{v.x, v.y, v.z, v.w};
+        }
       }
       if (kRB == 1) __syncthreads();  // the next row block refills the same buffer
     };
@@ -644,7 +650,8 @@ extern "C" int mxfp8_mlp_bwd(const void* gu, const void* xs, const void* xsT, co
   MX_CHECK_ARG(!dgu_out || q, "mxfp8_mlp_bwd: dgu_out needs q");
   if (wide) {
     if (r == 16) {
-      if (q) bwd_kernel<16, true, false, 2><<<grid, 512, 0, stm>>>(BWD_ARGS);
+      if (q && (q_layout & 3) == 3) bwd_kernel<16, true, false, 2, true><<<grid, 512, 0, stm>>>(BWD_ARGS);
+      else if (q) bwd_kernel<16, true, false, 2><<<grid, 512, 0, stm>>>(BWD_ARGS);
       else bwd_kernel<16, false, false, 2><<<grid, 512, 0, stm>>>(BWD_ARGS);
     } else {
       if (q) bwd_kernel<32, true, false, 2><<<grid, 512, 0, stm>>>(BWD_ARGS);
