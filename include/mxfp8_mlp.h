@@ -100,9 +100,9 @@ int mxfp8_dequant(const void* q, int64_t rows, int64_t cols, int64_t ld_q, const
  * layout bits: MXFP8_GEMM_A_TILED = A codes in the MX-tiled layout (mxfp8_quant_tiled / mxfp8_tile_codes,
  * lda ignored), MXFP8_GEMM_B_TILED = the same for B (results are bit-identical to row-major operands; the
  * tiled layout lets every DMA of the GEMM move a contiguous 1 KB instead of sixteen 64-byte row pieces);
- * MXFP8_GEMM_WIDE = 8-wave 256 x 256 workgroups, one per CU, instead of the default 4-wave 256 x 128, two per
- * CU (same result bits when no tile is split); MXFP8_GEMM_C_FT = C in the fused-tile (FT) layout instead of
- * row-major (ldc ignored; c holds ceil(M/32)*32 rows, rows past M not written).
+ * MXFP8_GEMM_WIDE = 8-wave 256 x 256 workgroups, one per CU; without it the workgroup shape (64 x 64 to 256 x 256)
+ * follows the size (same result bits when no tile is split); MXFP8_GEMM_C_FT = C in the fused-tile (FT) layout
+ * instead of row-major (ldc ignored; c holds ceil(M/32)*32 rows, rows past M not written).
  * FT layout of a bf16 [R, C] matrix (C % 32 == 0): 32 x 32 blocks of 2 KB, block (r/32, c/32) at
  * ((r/32) * (C/32) + c/32) * 1024 elements; element (r, c) inside it at ((c/8) % 2) * 512 +
  * (r%32 + 32 * ((c/16) % 2)) * 8 + c % 8.  It is the order in which the fused kernels' waves read a 32 x 32 tile
@@ -127,8 +127,8 @@ int mxfp8_gemm_nt(const void* a, const void* sa, int64_t lda, const void* b, con
 /*
  * mxfp8_gemm_nt with the output columns in n_seg (1..4) separate row-major matrices: columns
  * [seg_col0[k], seg_col0[k+1]) (the last up to N) go to seg_c[k] with row stride seg_ldc[k]; seg_col0[0] = 0 and
- * every boundary a multiple of 128.  seg_col0, seg_c and seg_ldc are host arrays.  The 4-wave shape with row-major
- * C only (layout bits 0-1), no workspace.  Lets the q|k|v projections of a group run as one GEMM over their
+ * every boundary a multiple of 128.  seg_col0, seg_c and seg_ldc are host arrays.  Row-major C in a
+ * 4-wave shape only (layout bits 0-1), no workspace.  Lets the q|k|v projections of a group run as one GEMM over their
  * concatenated weight while each returns its own contiguous output (the reference runs one _scaled_mm per layer,
  * /root/reference/scripts/fused_linear.py:72-76, :106-109).
  * seg_rcol (host array, or NULL for columns [0, r) everywhere): segment k adds the rank-r product over columns
@@ -428,10 +428,10 @@ int mxfp8_lora_tn_batch(const mxfp8_lora_tn_job* jobs, int64_t n_jobs, int64_t T
                         float* part, void* stream);
 
 /*
- * mxfp8_gemm_nt (4-wave shape, rank-16, 32 or 48 LoRA epilogue, no workspace) and mxfp8_lora_tn_batch in one
- * launch plus the batch's sums: the token reductions run in workgroups numbered after every GEMM tile, so the
- * dispatcher starts them only once each tile has started, in the workgroup slots the GEMM's last round of tiles
- * leaves idle.  Results bit for bit those of the two calls one after the other (jobs, T_tn, K_tn, chunks and part
+ * mxfp8_gemm_nt (rank-16, 32 or 48 LoRA epilogue, no workspace) and mxfp8_lora_tn_batch in one launch plus the
+ * batch's sums (two launches plus the sums for sizes that take the 8-wave shape): the token reductions run in
+ * workgroups numbered after every GEMM tile, so the dispatcher starts them only once each tile has started, in the
+ * workgroup slots the GEMM's last round of tiles leaves idle.  Results bit for bit those of the two calls one after the other (jobs, T_tn, K_tn, chunks and part
  * as in mxfp8_lora_tn_batch).  The jobs must not read c.  Replaces, in the MLP backward, the dx GEMM with its
  * dxa·S addmm_ and the token GEMMs dB_d, dA (/root/reference/scripts/fused_mlp.py:331, :316-318, :333), and in
  * the grouped linears' backward the dx GEMM with its dS·S addmm_ and dA = dSᵀ·x2 (fused_linear.py:269, :271), which
@@ -444,7 +444,7 @@ int mxfp8_gemm_nt_tn(const void* a, const void* sa, int64_t lda, const void* b, 
                      float* part, void* stream);
 
 /*
- * mxfp8_gemm_nt (4-wave shape, rank-16 LoRA epilogue, no workspace) whose epilogue operand P is summed in the same
+ * mxfp8_gemm_nt (rank-16 LoRA epilogue, no workspace) whose epilogue operand P is summed in the same
  * launch: P [M, r] (lora_p, row stride r, written) = bf16(part_scale · Σ_p part[p]) over the n_parts fp32 partials
  * part [n_parts, M, r], p ascending, exactly as mxfp8_sum_parts computes it.  Workgroups numbered before the
  * GEMM's tiles compute P and publish each block of rows; a tile waits for its rows only at its epilogue.  A tile

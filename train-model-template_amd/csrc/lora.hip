@@ -537,8 +537,8 @@ __device__ __forceinline__ void lora_bwd_body(const uint16_t* __restrict__ dy, i
       // (lanes l and l + 32 store the same word)
       // Tiled is what the dx GEMM reads: with row-major codes its 64-byte row pieces use half of each line per request
       // (q|k|v dx with its reduction at T = 10752, K = 3072: 107 -> 92 us, o_proj's, K = 2048: 73 -> 64; this kernel the
-      // same within 1 us).  In the MX-tiled layout (ld_q = its columns) the block is four contiguous 1 KB blocks of it: store j takes row
-      // half j / 2 and column half j % 2, lane l row l / 4 of it at 16-byte position l % 4.
+      // same within 1 us).  In the MX-tiled layout (ld_q = its columns) the block is four contiguous 1 KB blocks of it:
+      // store j takes row half j / 2 and column half j % 2, lane l row l / 4 of it at 16-byte position l % 4.
       const int64_t qc = (int64_t)col_tile_off * 128 + c0;
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -673,7 +673,8 @@ __global__ __launch_bounds__(256, 2) void lora_bwd_batch_kernel(const LoraBwdBat
 // The partials are read once: streaming (non-temporal) loads.  The backward finish at configuration 3 (graph timing,
 // one box, three alternating pairs, bit-identical): 13.07-13.10 us with plain loads, 12.01-12.03 us with these;
 // lora_bwd's sums unchanged (23.7 / 57.9 us with the main kernel).  Six in flight: the finish at T = 1000 / 10752 /
-// 142336 takes 6.2 / 12.3 / 169 us, with eight 5.9 / 12.9 / 172, with four 6.6 / 12.2 / 169.  (The forward's sum_parts kernel measured slower with them: 12.8 against 11.6 us.)
+// 142336 takes 6.2 / 12.3 / 169 us, with eight 5.9 / 12.9 / 172, with four 6.6 / 12.2 / 169.  (The forward's
+// sum_parts kernel measured slower with streaming loads: 12.8 against 11.6 us.)
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 __device__ __forceinline__ float4 ld_part(const float4* p) {
   const f32x4 t = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(p));

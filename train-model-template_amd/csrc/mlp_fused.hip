@@ -187,9 +187,9 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFwdWavesPe
 //     the super-block in registers and stored after it.
 // The large operands of the next row block (gu, dhm) are loaded one row block ahead.  The small per-row operands
 // (xs, dxd and their transposed copies, L2-resident; the same 6 r / 16 KB for every wave of the workgroup):
-//   r = 16, and r = 32 with 8 waves (kStage): staged in LDS one row block ahead, by global_load_lds DMAs issued at the start of the row
-//     block before (each 1 KB DMA lands as the lane-ordered MFMA operand, so the reads are conflict-free
-//     ds_read_b128), one copy per workgroup instead of one per wave.  Each wave drains its memory counter before
+//   r = 16, and r = 32 with 8 waves (kStage): staged in LDS one row block ahead, by global_load_lds DMAs issued at
+//     the start of the row block before (each 1 KB DMA lands as the lane-ordered MFMA operand, so the reads are
+//     conflict-free ds_read_b128), one copy per workgroup instead of one per wave.  Each wave drains its memory counter before
 //     the row block's barrier, and the block's code, scale and partial stores are issued after that barrier:
 //     the memory counter completes in issue order, so a wait for a load issued behind a store also waits for
 //     the store, and the previous form's first wait of every row block (for the small loads, issued behind the

@@ -24,12 +24,13 @@
 // (barrier, fragment reads, their wait: about 0.13 us, whatever the ring's depth) besides its MFMAs, so a launch of
 // few tiles takes (K steps) x (0.30, 0.23, 0.15, 0.12 us) at 256 x 128, 128 x 128, 64 x 128, 64 x 64, and Low and
 // Small take 128-wide K steps, half the barriers.  Long launches take Wide, which reads a third less per flop from
-// L2.  pick_shape chooses.
+// L2.  A Tall launch whose last tiles would run alone on their CUs gives those rows to Mid or Low tiles in the same
+// launch (its tail).  pick_shape chooses.
 //
-// What bounds it (rocprofv3 counters on the MLP GEMMs): the CU's vector-memory path that carries the
-// operand DMA (TA / TD busy 65-89% of the kernel, TD waiting on L1/L2 data about 45% of the time) while the
-// matrix pipe is busy ~48%.  LDS reads overlap MFMAs well on gfx950 (a software-pipelined fragment-read +
-// MFMA loop runs at 94-97% of the MFMA-only rate), and an L2 prefetch ahead of the ring made it slower.
+// What bounds it (rocprofv3 counters): with this order the matrix pipe is busy 71% (Tall) to 74% (Wide) of a long
+// launch at 1.72 and 1.52 GHz, so the power limit holds it; products of a step in serpentine order, which keep one
+// operand from each to the next, gained 0.3-0.8% there.  Before, the CU's vector-memory path that carries the operand
+// DMA held it (TA / TD busy 65-89%) at a matrix pipe busy ~48%.  An L2 prefetch ahead of the ring made it slower.
 //
 // Operand layouts: row-major codes (row stride lda / ldb), or the MX-tiled layout (tiled_offset in
 // mx_device.h) in which each 16-row x 64-code slice is one contiguous 1 KB block in LDS order.  The GEMM is
@@ -1408,7 +1409,8 @@ extern "C" int mxfp8_gemm_swiglu_fwd(const void* a, const void* sa, const void* 
   const uint8_t *A = (const uint8_t*)a, *SA = (const uint8_t*)sa, *B = (const uint8_t*)b, *SB = (const uint8_t*)sb;
 #define SWIGLU_LAUNCH(R, S)                                                                                        \
   gemm_kernel<R, S, kEpiSwiGluFwd><<<grid, S::kThreads, 0, stm>>>(A, SA, K, B, SB, K, (int)M, (int)(2 * N), (int)K, cs, \
-                                                                  Lora{}, plan, tiled, sw, SwBwd{}, TnBatch{}, PreSum{}, Plan{})
+                                                                  Lora{}, plan, tiled, sw, SwBwd{}, TnBatch{}, PreSum{}, \
+                                                                  Plan{})
   if (mid) {
     if (r == 16) SWIGLU_LAUNCH(16, Mid);
     else SWIGLU_LAUNCH(32, Mid);

@@ -484,8 +484,8 @@ def _native_per_layer(spec, x2, xS, flat, dt):
 def _native_backward(spec, skey, x2, xS, S, Bs, flat, slots, need_x):
     """_plain_backward on the library's kernels: per layer one read of dy for its MX codes, d(xa) and dB (fp32, not
     rounded to bf16 first) and one MX GEMM for its dgrad, the last with dS·S in its epilogue and dA's token
-    reduction in its launch.  At T = 2688, d_model 1024, d_ffn 3584 the two groups of an MLP took 36 launches and 398 us of kernels
-    a step with the skinny products on the BLAS library (19-25 us each); here 21 launches and 264 us."""
+    reduction in its launch.  At T = 2688, d_model 1024, d_ffn 3584 the two groups of an MLP took 36 launches and
+    398 us of kernels a step with the skinny products on the BLAS library (19-25 us each); here 21 launches and 264 us."""
     import _native
     import mxfp8
     T = x2.shape[0]
