@@ -421,7 +421,7 @@ class _Group(torch.autograd.Function):
             dx, grads = _fused_backward(spec, ctx.skey, x2, xS, S, Bs, flat, plan, need_x, dt)
             STATS["lan ngược gộp"] = STATS.get("lan ngược gộp", 0) + 1
         else:
-            slots = _native_per_layer(spec, x2, xS, flat, dt)
+            slots = _native_per_layer(spec, x2, xS, Bs, flat, dt)
             if slots is not None:
                 dx, grads = _native_backward(spec, ctx.skey, x2, xS, S, Bs, flat, slots, need_x)
             else:
@@ -470,13 +470,17 @@ def _tn_job(x2, dS, width, out_dtype):
     return (x2, dS, out, 1.0, False), part
 
 
-def _native_per_layer(spec, x2, xS, flat, dt):
+def _native_per_layer(spec, x2, xS, Bs, flat, dt):
     """The adapter slots when the per-layer backward runs on the library's kernels (_native_backward): bf16 math,
     only MX layers, each with an adapter of one common rank 16 or 32 and a gradient, at most 64 rank columns.  These
-    are the MLP's projections outside the fused MLP, which have no concatenated Wᵀ."""
+    are the MLP's projections outside the fused MLP, which have no concatenated Wᵀ.  The kernels index B as
+    [N, r] contiguous; a cast keeps its parameter's strides (a transposed fp64 or fp16 B), and such a B stays with the
+    torch products."""
     if dt != torch.bfloat16 or spec.thin or spec.plain or not spec.mx or len(spec.mx) != len(spec.adapters):
         return None
     if not _native_ok(x2, dt, spec.width) or any(dy is None for dy in flat):
+        return None
+    if not all(b.is_contiguous() and b.dtype == dt for b in Bs):
         return None
     return _lora_bwd_batchable(spec, flat, xS)
 
