@@ -421,11 +421,7 @@ class _Group(torch.autograd.Function):
             dx, grads = _fused_backward(spec, ctx.skey, x2, xS, S, Bs, flat, plan, need_x, dt)
             STATS["lan ngược gộp"] = STATS.get("lan ngược gộp", 0) + 1
         else:
-            slots = _native_per_layer(spec, x2, xS, Bs, flat, dt)
-            if slots is not None:
-                dx, grads = _native_backward(spec, ctx.skey, x2, xS, S, Bs, flat, slots, need_x)
-            else:
-                dx, grads = _plain_backward(spec, x2, xS, S, Bs, flat, need_x, dt)
+            dx, grads = _plain_backward(spec, x2, xS, S, Bs, flat, need_x, dt)
         # A / B may be fp32 parameters while the math runs in bf16: autograd casts the gradients to their dtype
         wanted = ctx.needs_input_grad[4:]
         grads = [g if (g is not None and wanted[k]) else None for k, g in enumerate(grads)]
@@ -468,58 +464,6 @@ def _tn_job(x2, dS, width, out_dtype):
     n_part = _native.lora_tn_chunks(T, K) * width * K
     part = _native.scratch_f32(n_part, x2.device)[:n_part]  # partial sums, read by the launch's sum kernel
     return (x2, dS, out, 1.0, False), part
-
-
-def _native_per_layer(spec, x2, xS, Bs, flat, dt):
-    """The adapter slots when the per-layer backward runs on the library's kernels (_native_backward): bf16 math,
-    only MX layers, each with an adapter of one common rank 16 or 32 and a gradient, at most 64 rank columns.  These
-    are the MLP's projections outside the fused MLP, which have no concatenated Wᵀ.  The kernels index B as
-    [N, r] contiguous; a cast keeps its parameter's strides (a transposed fp64 or fp16 B), and such a B stays with the
-    torch products."""
-    if dt != torch.bfloat16 or spec.thin or spec.plain or not spec.mx or len(spec.mx) != len(spec.adapters):
-        return None
-    if not _native_ok(x2, dt, spec.width) or any(dy is None for dy in flat):
-        return None
-    if not all(b.is_contiguous() and b.dtype == dt for b in Bs):
-        return None
-    return _lora_bwd_batchable(spec, flat, xS)
-
-
-def _native_backward(spec, skey, x2, xS, S, Bs, flat, slots, need_x):
-    """_plain_backward on the library's kernels: per layer one read of dy for its MX codes, d(xa) and dB (fp32, not
-    rounded to bf16 first) and one MX GEMM for its dgrad, the last with dS·S in its epilogue and dA's token
-    reduction in its launch.  At T = 2688, d_model 1024, d_ffn 3584 the two groups of an MLP took 36 launches and
-    398 us of kernels a step with the skinny products on the BLAS library (19-25 us each); here 21 launches and 264 us."""
-    import _native
-    import mxfp8
-    T = x2.shape[0]
-    rp, stream = _rp(spec.width), _native.stream_of(x2)
-    dS = torch.empty((T, rp), dtype=torch.bfloat16, device=x2.device)
-    r_dx = spec.width if spec.width in (16, 32, 48, 64) else rp
-    if r_dx > spec.width:
-        dS[:, spec.width:].zero_()
-    grads, dx = [None] * (2 * len(slots)), None
-    a32 = all(spec.parts[i][1].dtype == torch.float32 for i in spec.mx)
-    job, part = _tn_job(x2, dS, rp, torch.float32 if a32 else torch.bfloat16)
-    fold = need_x and FOLD_TN[0] and r_dx in (16, 32, 48)  # dA in the last dx GEMM's launch
-    for sl, i in zip(slots, spec.mx):
-        q, s, (grads[2 * sl.index + 1],) = _native.host().group_lora_bwd([flat[i]], xS, [Bs[sl.index]], [sl.col],
-                                                                         [sl.scale], dS, need_x, stream)
-        if need_x:
-            wq, ws, lay = mxfp8.group_operand([spec.parts[i][0]])
-            lay |= _native.GEMM_A_TILED
-            if i != spec.mx[-1]:
-                g = mxfp8.mx_mm(q, s, wq, ws, layout=lay, m=T)
-            else:
-                lora = (dS[:, :r_dx], _st(S, skey, rp)[:, :r_dx])
-                g = (mxfp8.mx_mm_tn(q, s, wq, ws, lora, 1.0, lay, T, [job], part) if fold
-                     else mxfp8.mx_mm(q, s, wq, ws, lora=lora, layout=lay, m=T))
-            dx = g if dx is None else dx.add_(g)
-    if not fold:
-        _native.lora_tn(x2, dS, job[2], part)
-    for sl in slots:
-        grads[2 * sl.index] = job[2][sl.cols]
-    return dx, grads
 
 
 def _plain_backward(spec, x2, xS, S, Bs, flat, need_x, dt):
