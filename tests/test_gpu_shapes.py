@@ -76,3 +76,29 @@ def test_folded_launches_in_every_shape(M, N, K, gpu):
     _native.lora_tn_batch([(x, P3, outs[0], 1.0, False)], scratch)
     got = mxfp8.mx_mm_tn(qa, sa, qb, sb, (P3, Q), 1.0, 3, M, [(x, P3, outs[1], 1.0, False)], scratch)
     assert torch.equal(outs[0], outs[1]) and torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("rank", [0, 16])
+@pytest.mark.parametrize("split", [False, True])
+@pytest.mark.parametrize("M,N,K", [(300, 384, 256), (257, 128, 512)])
+def test_the_8_wave_shape_past_the_last_column(M, N, K, split, rank, gpu):
+    """MXFP8_GEMM_WIDE | MXFP8_GEMM_B_PI with N % 256 == 128: the half of the last 256-column tile that lies past N is
+    not stored.  C row-major with guard columns (a tile's width of them) and guard rows, and in the fused-tile layout;
+    the same bits as without MXFP8_GEMM_B_PI, split along K or not."""
+    g, (qa, sa), (qb, sb), b = _operands(M, N, K, gpu)
+    qp, sp = mxfp8.mx_quant_tiled(b[mxfp8.fused_dgrad_rows(N, gpu)].contiguous())
+    lora = None
+    if rank:
+        lora = ((torch.randn(M, rank, device=gpu, generator=g) * 0.1).to(torch.bfloat16),
+                (torch.randn(N, rank, device=gpu, generator=g) * 0.1).to(torch.bfloat16))
+    got, want = (torch.full((M + 8, N + 256), 3.0, dtype=torch.bfloat16, device=gpu) for _ in range(2))
+    kw = dict(lora=lora, alpha=0.7, split=split)
+    _native.gemm_nt(qa, sa, K, qb, sb, K, M, N, K, want[:M, :N], layout=3 | _native.GEMM_WIDE, **kw)
+    _native.gemm_nt(qa, sa, K, qp, sp, K, M, N, K, got[:M, :N], layout=3 | _native.GEMM_WIDE | _native.GEMM_B_PI, **kw)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+    assert bool((got[:, N:] == 3.0).all()) and bool((got[M:] == 3.0).all())
+    ft = [torch.full((mxfp8.ft_rows(M) + 32, N), 3.0, dtype=torch.bfloat16, device=gpu) for _ in range(2)]
+    for c, q, s, bit in ((ft[0], qb, sb, 0), (ft[1], qp, sp, _native.GEMM_B_PI)):
+        _native.gemm_nt(qa, sa, K, q, s, K, M, N, K, c, layout=3 | _native.GEMM_WIDE | _native.GEMM_C_FT | bit, **kw)
+    assert torch.equal(ft[0].view(torch.int16), ft[1].view(torch.int16))
+    assert bool((ft[1][mxfp8.ft_rows(M):] == 3.0).all())

@@ -885,6 +885,9 @@ __device__ __forceinline__ void gemm_body(const uint8_t* __restrict__ A, const u
 #pragma unroll
   for (int nt = 0; nt < kNB; ++nt) {
     const int nb = n0 + (wn * kNB + nt) * 32;
+    // N % 128 == 0: only Wide's last tile column can lie past N, in whole waves
+    if constexpr (S::kBN > 128)
+      if (nb >= N) break;
     if constexpr (kR > 0) {
       if (nt + 1 < kNB) load_q(nt + 1, qf[(nt + 1) & 1]);
     }
@@ -913,7 +916,7 @@ __device__ __forceinline__ void gemm_body(const uint8_t* __restrict__ A, const u
         }
       }
       if (m >= M) continue;
-      if (b_pi) {  // columns nb + (lane/32)*16 + 0..15 (N % 128 == 0: all inside)
+      if (b_pi) {  // columns nb + (lane/32)*16 + 0..15
         const int n = nb + (lane >> 5) * 16;
         if (c_ft) {
           uint16_t* p = C + ft_offset(m, n, N);
@@ -929,9 +932,8 @@ __device__ __forceinline__ void gemm_body(const uint8_t* __restrict__ A, const u
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const int n = nb + g * 8 + (lane >> 5) * 4;
-        if (n < N)
-          *reinterpret_cast<uint2*>(C + (c_ft ? ft_offset(m, n, N) : (int64_t)m * ldc + (n - ncol0))) =
-              make_uint2(wv[2 * g], wv[2 * g + 1]);
+        *reinterpret_cast<uint2*>(C + (c_ft ? ft_offset(m, n, N) : (int64_t)m * ldc + (n - ncol0))) =
+            make_uint2(wv[2 * g], wv[2 * g + 1]);
       }
     }
   }
