@@ -7,13 +7,17 @@
 // Python wrappers of _native.py, so the same bits; temporaries that no tensor has to name share one allocation, cut
 // into 256-byte aligned pieces, which lives until its function returns (the caching allocator hands the memory on
 // only to later work of the same stream).  Shapes, dtypes and strides that the callers do not check themselves are
-// checked here; an error of the library raises _native.NativeError with its message.
+// checked here; an error of the library raises _native.NativeError with its message.  Every function runs without the
+// interpreter's lock, as a ctypes call does: a launch may wait for room in the stream's queue, and other Python threads
+// go on meanwhile.  Nothing below touches a Python object.
 // Counterpart of the Python glue of /root/reference/scripts/fused_mlp.py:262-336, mxfp8.py:78-293 and
 // fused_linear.py:219-279.
 #include <torch/extension.h>
 
 #include <array>
 #include <optional>
+#include <stdexcept>
+#include <string>
 #include <tuple>
 #include <vector>
 
@@ -34,10 +38,10 @@ int64_t ft_rows(int64_t r) { return cdiv(r, 32) * 32; }
 
 PyObject* g_error = nullptr;  // _native.NativeError
 
-[[noreturn]] void raise(const std::string& msg) {
-  PyErr_SetString(g_error ? g_error : PyExc_RuntimeError, msg.c_str());
-  throw py::error_already_set();
-}
+struct NativeError : std::runtime_error {  // becomes g_error in Python
+  using std::runtime_error::runtime_error;
+};
+[[noreturn]] void raise(const std::string& msg) { throw NativeError(msg); }
 void ok(int rc, const char* name) {
   if (rc) raise(std::string(name) + " failed with code " + std::to_string(rc) + ": " + mxfp8_last_error());
 }
@@ -357,17 +361,25 @@ PYBIND11_MODULE(_mxhost, m) {
     Py_XDECREF(g_error);
     g_error = e.ptr();
   });
+  py::register_local_exception_translator([](std::exception_ptr p) {
+    try {
+      if (p) std::rethrow_exception(p);
+    } catch (const NativeError& e) {
+      PyErr_SetString(g_error ? g_error : PyExc_RuntimeError, e.what());
+    }
+  });
   m.def("abi_version", [] { return MXFP8_MLP_ABI_VERSION; });
-  m.def("quant_rows", &quant_rows);
-  m.def("quant_tiled", &quant_tiled);
-  m.def("quant_lora", &quant_lora);
-  m.def("gemm", &gemm);
-  m.def("gemm_seg", &gemm_seg);
-  m.def("gemm_tn", &gemm_tn);
-  m.def("res_lora", &res_lora);
-  m.def("group_lora_bwd", &group_lora_bwd);
-  m.def("mlp_forms", &mlp_forms);
-  m.def("mlp_forward", &mlp_forward);
-  m.def("mlp_graph", &mlp_graph);
-  m.def("mlp_backward", &mlp_backward);
+  const auto def = [&m](const char* name, auto f) { m.def(name, f, py::call_guard<py::gil_scoped_release>()); };
+  def("quant_rows", &quant_rows);
+  def("quant_tiled", &quant_tiled);
+  def("quant_lora", &quant_lora);
+  def("gemm", &gemm);
+  def("gemm_seg", &gemm_seg);
+  def("gemm_tn", &gemm_tn);
+  def("res_lora", &res_lora);
+  def("group_lora_bwd", &group_lora_bwd);
+  def("mlp_forms", &mlp_forms);
+  def("mlp_forward", &mlp_forward);
+  def("mlp_graph", &mlp_graph);
+  def("mlp_backward", &mlp_backward);
 }
