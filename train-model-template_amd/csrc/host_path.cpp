@@ -4,9 +4,10 @@
 // Why: at a few thousand tokens and below a pass is bound by the host.  The launches themselves cost about 3 us each
 // on the host; the Python around them (an allocation 1.7 us, address and stride lookups, ctypes conversions and
 // structures) cost two to three times as much again.  Same launches in the same order on the same stream as the
-// Python wrappers of _native.py, so the same bits; temporaries that no tensor has to name share one allocation, cut
-// into 256-byte aligned pieces, which lives until its function returns (the caching allocator hands the memory on
-// only to later work of the same stream).  Shapes, dtypes and strides that the callers do not check themselves are
+// Python wrappers of _native.py, so the same bits; temporaries that no tensor has to name and that live as long as each
+// other share one allocation, cut into 256-byte aligned pieces (the caching allocator hands the memory on only to later
+// work of the same stream).  A pass holds no more memory at its peak than with one tensor for each: 142336 tokens,
+// 2048 x 6144, rank 16, 5.87 GB forward and 4.26 GB backward (6.17 and 5.18 GB with one allocation for all).  Shapes, dtypes and strides that the callers do not check themselves are
 // checked here; an error of the library raises _native.NativeError with its message.  Every function runs without the
 // interpreter's lock, as a ctypes call does: a launch may wait for room in the stream's queue, and other Python threads
 // go on meanwhile.  Nothing below touches a Python object.
@@ -14,6 +15,7 @@
 // fused_linear.py:219-279.
 #include <torch/extension.h>
 
+#include <algorithm>
 #include <array>
 #include <optional>
 #include <stdexcept>
@@ -58,7 +60,8 @@ Tensor empty(at::IntArrayRef shape, at::ScalarType dt, const Tensor& like) {
   return at::empty(shape, like.options().dtype(dt).requires_grad(false));
 }
 
-// One allocation for a call's temporaries: sizes are taken first (take), addresses once it is made (at).
+// One allocation for temporaries with one life: sizes are taken first (take), addresses once it is made (at).  drop()
+// hands the memory back for what is allocated next: the work is ordered by the stream, so its last reader may still run.
 struct Arena {
   int64_t total = 0;
   Tensor buf;
@@ -68,6 +71,7 @@ struct Arena {
     return off;
   }
   void make(const Tensor& like) { buf = empty({total}, at::kByte, like); }
+  void drop() { buf.reset(); }
   void* at(int64_t off) const { return static_cast<char*>(buf.data_ptr()) + off; }
   float* f(int64_t off) const { return static_cast<float*>(at(off)); }
 };
@@ -253,28 +257,42 @@ std::tuple<Tensor, Tensor, Tensor> mlp_forward(const Tensor& x, const Tensor& S,
                                                int64_t fold_sum, int64_t stream) {
   gpu(x, "mxfp8_gemm_swiglu_fwd");
   const int64_t T = x.size(0), K = x.size(1), R = ad.size(0), N = ad.size(1);
-  Tensor xs = empty({T, 2 * R}, kBF, x), gu = empty({ft_rows(T), 2 * N}, kBF, x), y = empty({T, wd.size(0)}, kBF, x);
-  Arena a;
-  const int64_t q = a.take(tiled_rows(T) * K), s = a.take(scale_numel(T, K)), qh = a.take(tiled_rows(T) * N),
-                sh = a.take(scale_numel(T, N)), part = a.take(2 * N / 128 * T * R * 4), xsd = a.take(T * R * 2);
+  Tensor xs = empty({T, 2 * R}, kBF, x), gu = empty({ft_rows(T), 2 * N}, kBF, x), y;
+  const int64_t parts = 2 * N / 128;
+  const bool fold = R == 16 && T * R <= fold_sum;
+  // a: the codes of x, dropped after the gate|up GEMM; b: the codes of h; the xS_down partials and their sum in b where the
+  // down GEMM makes it, else the partials in c, dropped after their sum
+  Arena a, b, c;
+  Arena& p = fold ? b : c;
+  const int64_t q = a.take(tiled_rows(T) * K), s = a.take(scale_numel(T, K));
+  const int64_t qh = b.take(tiled_rows(T) * N), sh = b.take(scale_numel(T, N)), part = p.take(parts * T * R * 4),
+                xsd_b = fold ? b.take(T * R * 2) : 0;
   a.make(x);
+  b.make(x);
+  if (!fold) c.make(x);
   ok(mxfp8_quant_lora(ptr(x), T, K, x.stride(0), a.at(q), a.at(s), ptr(S), 2 * R, 1.f, ptr(xs), nullptr,
                       cdiv(T, 128) * 128, stm(stream)),
      "mxfp8_quant_lora");
   ok(mxfp8_gemm_swiglu_fwd(a.at(q), a.at(s), ptr(wf), ptr(wfs), T, N, K, ptr(xs), ptr(bg), ptr(bu), ptr(ad), R,
-                           (float)s_g, (float)s_u, ptr(gu), a.at(qh), a.at(sh), a.f(part), stm(stream)),
+                           (float)s_g, (float)s_u, ptr(gu), b.at(qh), b.at(sh), p.f(part), stm(stream)),
      "mxfp8_gemm_swiglu_fwd");
-  const int64_t lay = MXFP8_GEMM_A_TILED | MXFP8_GEMM_B_TILED | MXFP8_GEMM_B_PI, parts = 2 * N / 128;
-  if (R == 16 && T * R <= fold_sum) {
-    ok(mxfp8_gemm_nt_sum(a.at(qh), a.at(sh), N, ptr(wd), ptr(wds), N, T, wd.size(0), N, ptr(y), y.stride(0), a.f(part),
-                         parts, 1.f, a.at(xsd), ptr(bd), bd.stride(0), R, (float)s_d, lay, -1, stm(stream)),
+  a.drop();
+  Tensor xsd;
+  if (!fold) {
+    xsd = empty({T, R}, kBF, x);
+    ok(mxfp8_sum_parts(c.f(part), parts, T * R, 1.f, ptr(xsd), 1, stm(stream)), "mxfp8_sum_parts");
+    c.drop();
+  }
+  y = empty({T, wd.size(0)}, kBF, x);
+  const int64_t lay = MXFP8_GEMM_A_TILED | MXFP8_GEMM_B_TILED | MXFP8_GEMM_B_PI;
+  if (fold)
+    ok(mxfp8_gemm_nt_sum(b.at(qh), b.at(sh), N, ptr(wd), ptr(wds), N, T, wd.size(0), N, ptr(y), y.stride(0), b.f(part),
+                         parts, 1.f, b.at(xsd_b), ptr(bd), bd.stride(0), R, (float)s_d, lay, -1, stm(stream)),
        "mxfp8_gemm_nt_sum");
-  } else {
-    ok(mxfp8_sum_parts(a.f(part), parts, T * R, 1.f, a.at(xsd), 1, stm(stream)), "mxfp8_sum_parts");
-    ok(mxfp8_gemm_nt(a.at(qh), a.at(sh), N, ptr(wd), ptr(wds), N, T, wd.size(0), N, ptr(y), y.stride(0), a.at(xsd), R,
+  else
+    ok(mxfp8_gemm_nt(b.at(qh), b.at(sh), N, ptr(wd), ptr(wds), N, T, wd.size(0), N, ptr(y), y.stride(0), ptr(xsd), R,
                      ptr(bd), bd.stride(0), R, (float)s_d, lay, nullptr, 0, stm(stream)),
        "mxfp8_gemm_nt");
-  }
   return {y, xs, gu};
 }
 
@@ -307,46 +325,58 @@ std::tuple<OptT, Tensor, Tensor, Tensor, Tensor, Tensor> mlp_backward(
   const Tensor &ST = f[1], &bg = f[2], &bu = f[3], &bgT = f[4], &buT = f[5], &ad = f[6], &adT = f[7], &bdT = f[9];
   const int64_t T = dy.size(0), K = x.size(1), R = ad.size(0), N = ad.size(1), tpad = cdiv(T, 128) * 128;
   const int64_t nsb = cdiv(tpad, SB), n_dxa = N / (wide ? 256 : 128), chunks = mxfp8_lora_tn_chunks(T, K);
-  Tensor dA = empty({2 * R, K}, fp32_a ? kF32 : kBF, dy), dBg = empty({N, R}, kF32, dy), dBu = empty({N, R}, kF32, dy),
-         dAd = empty({R, N}, kF32, dy), dBd = empty({K, R}, fp32_bd ? kF32 : kBF, dy);
-  OptT dx;
-  if (need_x) dx = empty({T, K}, kBF, dy);
-  Arena a;
-  const int64_t qd = a.take(tiled_rows(T) * dy.size(1)), sd = a.take(scale_numel(T, dy.size(1))), dxd = a.take(T * R * 2),
-                dxdT = a.take(R * tpad * 2), xsT = a.take(2 * R * tpad * 2), dhm = a.take(ft_rows(T) * N * 2),
-                qg = need_x ? a.take(tiled_rows(T) * 2 * N) : 0, sg = need_x ? a.take(scale_numel(T, 2 * N)) : 0,
-                dxa_p = a.take(n_dxa * T * 3 * R * 4), dbg_p = a.take(nsb * N * R * 4), dbu_p = a.take(nsb * N * R * 4),
-                dad_p = a.take(nsb * R * N * 4), dxa = a.take(T * 2 * R * 2), xsd = a.take(T * R * 2),
-                part = a.take(chunks * 3 * R * K * 4);
+  // a: until the finish, the codes of dy (read by the dh GEMM) under the partials (written after it); m: dhm; b: the
+  // codes of dg | du; c: the finish's results; d: the token reductions' partials, made once a is dropped
+  Arena a, m, b, c, d;
+  const int64_t dxd = a.take(T * R * 2), dxdT = a.take(R * tpad * 2), xsT = a.take(2 * R * tpad * 2);
+  const int64_t under = a.total, qd = a.take(tiled_rows(T) * dy.size(1)), sd = a.take(scale_numel(T, dy.size(1)));
+  const int64_t codes_end = a.total;
+  a.total = under;
+  const int64_t dxa_p = a.take(n_dxa * T * 3 * R * 4), dbg_p = a.take(nsb * N * R * 4), dbu_p = a.take(nsb * N * R * 4),
+                dad_p = a.take(nsb * R * N * 4);
+  a.total = std::max(a.total, codes_end);
+  const int64_t dhm = m.take(ft_rows(T) * N * 2);
+  const int64_t qg = need_x ? b.take(tiled_rows(T) * 2 * N) : 0, sg = need_x ? b.take(scale_numel(T, 2 * N)) : 0;
+  const int64_t dxa = c.take(T * 2 * R * 2), xsd = c.take(T * R * 2), part = d.take(chunks * 3 * R * K * 4);
   a.make(dy);
+  m.make(dy);
   void* const st = stm(stream);
   ok(mxfp8_quant_lora_tp(ptr(dy), T, dy.size(1), dy.stride(0), a.at(qd), a.at(sd), ptr(bdT), R, (float)s_d, a.at(dxd),
                          a.at(dxdT), tpad, ptr(xs), xs.stride(0), 2 * R, a.at(xsT), st),
      "mxfp8_quant_lora_tp");
   const int64_t tt = MXFP8_GEMM_A_TILED | MXFP8_GEMM_B_TILED;
-  ok(mxfp8_gemm_nt(a.at(qd), a.at(sd), dy.size(1), ptr(wt), ptr(wts), dy.size(1), T, N, dy.size(1), a.at(dhm), N, nullptr,
+  ok(mxfp8_gemm_nt(a.at(qd), a.at(sd), dy.size(1), ptr(wt), ptr(wts), dy.size(1), T, N, dy.size(1), m.at(dhm), N, nullptr,
                    0, nullptr, 0, 0, 1.f, tt | MXFP8_GEMM_C_FT | MXFP8_GEMM_B_PI, nullptr, 0, st),
      "mxfp8_gemm_nt");
-  ok(mxfp8_mlp_bwd(ptr(gu), ptr(xs), a.at(xsT), a.at(dhm), a.at(dxd), a.at(dxdT), ptr(bg), ptr(bu), ptr(bgT), ptr(buT),
-                   ptr(ad), ptr(adT), T, N, R, (float)s_g, (float)s_u, SB, CG, need_x ? a.at(qg) : nullptr,
-                   need_x ? a.at(sg) : nullptr, a.f(dxa_p), a.f(dbg_p), a.f(dbu_p), a.f(dad_p), nullptr,
+  if (need_x) b.make(dy);
+  ok(mxfp8_mlp_bwd(ptr(gu), ptr(xs), a.at(xsT), m.at(dhm), a.at(dxd), a.at(dxdT), ptr(bg), ptr(bu), ptr(bgT), ptr(buT),
+                   ptr(ad), ptr(adT), T, N, R, (float)s_g, (float)s_u, SB, CG, need_x ? b.at(qg) : nullptr,
+                   need_x ? b.at(sg) : nullptr, a.f(dxa_p), a.f(dbg_p), a.f(dbu_p), a.f(dad_p), nullptr,
                    1 | 2 | (wide ? 4 : 0), st),
      "mxfp8_mlp_bwd");
+  m.drop();
+  c.make(dy);
+  Tensor dA = empty({2 * R, K}, fp32_a ? kF32 : kBF, dy), dBg = empty({N, R}, kF32, dy), dBu = empty({N, R}, kF32, dy),
+         dAd = empty({R, N}, kF32, dy), dBd = empty({K, R}, fp32_bd ? kF32 : kBF, dy);
   ok(mxfp8_mlp_bwd_finish(a.f(dxa_p), a.f(dbg_p), a.f(dbu_p), a.f(dad_p), n_dxa, nsb, T, N, R, (float)s_g, (float)s_u,
-                          a.at(dxa), a.at(xsd), fptr(dBg), fptr(dBu), fptr(dAd), st),
+                          c.at(dxa), c.at(xsd), fptr(dBg), fptr(dBu), fptr(dAd), st),
      "mxfp8_mlp_bwd_finish");
-  const mxfp8_lora_tn_job jobs[2] = {{ptr(dy), dy.stride(0), a.at(xsd), R, (float)s_d, 1, fp32_bd, ptr(dBd)},
-                                     {ptr(x), x.stride(0), a.at(dxa), 2 * R, 1.f, 0, fp32_a, ptr(dA)}};
+  a.drop();
+  d.make(dy);
+  const mxfp8_lora_tn_job jobs[2] = {{ptr(dy), dy.stride(0), c.at(xsd), R, (float)s_d, 1, fp32_bd, ptr(dBd)},
+                                     {ptr(x), x.stride(0), c.at(dxa), 2 * R, 1.f, 0, fp32_a, ptr(dA)}};
   const bool fold = need_x && R == 16;
-  if (!fold) ok(mxfp8_lora_tn_batch(jobs, 2, T, K, chunks, a.f(part), st), "mxfp8_lora_tn_batch");
+  if (!fold) ok(mxfp8_lora_tn_batch(jobs, 2, T, K, chunks, d.f(part), st), "mxfp8_lora_tn_batch");
+  OptT dx;
   if (need_x) {
+    dx = empty({T, K}, kBF, dy);
     const int64_t lay = tt | MXFP8_GEMM_B_PI;
     if (fold)
-      ok(mxfp8_gemm_nt_tn(a.at(qg), a.at(sg), 2 * N, ptr(wx), ptr(wxs), 2 * N, T, K, 2 * N, ptr(dx), K, a.at(dxa), 2 * R,
-                          ptr(ST), ST.stride(0), 2 * R, 1.f, lay, jobs, 2, T, K, chunks, a.f(part), st),
+      ok(mxfp8_gemm_nt_tn(b.at(qg), b.at(sg), 2 * N, ptr(wx), ptr(wxs), 2 * N, T, K, 2 * N, ptr(dx), K, c.at(dxa), 2 * R,
+                          ptr(ST), ST.stride(0), 2 * R, 1.f, lay, jobs, 2, T, K, chunks, d.f(part), st),
          "mxfp8_gemm_nt_tn");
     else
-      ok(mxfp8_gemm_nt(a.at(qg), a.at(sg), 2 * N, ptr(wx), ptr(wxs), 2 * N, T, K, 2 * N, ptr(dx), K, a.at(dxa), 2 * R,
+      ok(mxfp8_gemm_nt(b.at(qg), b.at(sg), 2 * N, ptr(wx), ptr(wxs), 2 * N, T, K, 2 * N, ptr(dx), K, c.at(dxa), 2 * R,
                        ptr(ST), ST.stride(0), 2 * R, 1.f, lay, nullptr, 0, st),
          "mxfp8_gemm_nt");
   }
