@@ -189,8 +189,22 @@ std::tuple<OptT, OptT, std::vector<Tensor>> group_lora_bwd(const std::vector<Ten
                                                            const std::vector<int64_t>& cols,
                                                            const std::vector<double>& scales, const Tensor& dS,
                                                            bool need_q, int64_t stream) {
-  const int64_t n = (int64_t)dys.size(), T = dys[0].size(0), R = Bs[0].size(1);
-  TORCH_CHECK(n >= 1 && n <= MXFP8_LORA_BWD_MAX_JOBS && T > 0, "group_lora_bwd: 1 to 8 layers, T > 0");
+  const int64_t n = (int64_t)dys.size();
+  TORCH_CHECK(n >= 1 && n <= MXFP8_LORA_BWD_MAX_JOBS && (int64_t)Bs.size() == n && (int64_t)cols.size() == n &&
+                  (int64_t)scales.size() == n && dys[0].size(0) > 0,
+              "group_lora_bwd: 1 to 8 layers, T > 0");
+  const int64_t T = dys[0].size(0), R = Bs[0].size(1);
+  TORCH_CHECK(xS.scalar_type() == kBF && dS.scalar_type() == kBF && xS.stride(1) == 1 && dS.stride(1) == 1 &&
+                  xS.size(0) == T && dS.size(0) == T,
+              "group_lora_bwd: xS and dS [T, *] bf16 with unit column stride");
+  for (int64_t k = 0; k < n; ++k) {
+    const int64_t N = dys[k].size(1);
+    TORCH_CHECK(dys[k].scalar_type() == kBF && dys[k].size(0) == T && dys[k].stride(1) == 1 && N % 128 == 0 &&
+                    Bs[k].is_contiguous() && Bs[k].size(0) == N && Bs[k].size(1) == R && Bs[k].scalar_type() == kBF,
+                "group_lora_bwd: dy [T, N] bf16 with unit column stride, N % 128 == 0, and B [N, r] bf16 contiguous");
+    TORCH_CHECK(cols[k] >= 0 && cols[k] + R <= xS.size(1) && cols[k] + R <= dS.size(1),
+                "group_lora_bwd: columns ", cols[k], " to ", cols[k] + R, " of xS and dS");
+  }
   gpu(dys[0], "mxfp8_lora_bwd");
   int64_t sum_n = 0;
   for (const auto& d : dys) sum_n += d.size(1);
@@ -205,16 +219,10 @@ std::tuple<OptT, OptT, std::vector<Tensor>> group_lora_bwd(const std::vector<Ten
   std::vector<Tensor> dbs;
   for (int64_t k = 0; k < n; ++k) {
     const int64_t N = dys[k].size(1);
-    TORCH_CHECK(dys[k].scalar_type() == kBF && dys[k].size(0) == T && dys[k].stride(1) == 1 && N % 128 == 0 &&
-                    Bs[k].is_contiguous() && Bs[k].size(0) == N && Bs[k].size(1) == R && Bs[k].scalar_type() == kBF,
-                "group_lora_bwd: dy [T, N] bf16 with unit column stride, N % 128 == 0, and B [N, r] bf16 contiguous");
     pdx[k] = a.take(N / 128 * T * R * 4);
     pdb[k] = a.take(chunks * N * R * 4);
     dbs.push_back(empty({N, R}, kF32, dys[k]));
   }
-  TORCH_CHECK(xS.scalar_type() == kBF && dS.scalar_type() == kBF && xS.stride(1) == 1 && dS.stride(1) == 1 &&
-                  xS.size(0) == T && dS.size(0) == T,
-              "group_lora_bwd: xS and dS [T, *] bf16 with unit column stride");
   a.make(dys[0]);
   auto* xs = static_cast<uint16_t*>(xS.data_ptr());
   auto* ds = static_cast<uint16_t*>(dS.data_ptr());
@@ -232,6 +240,12 @@ std::tuple<OptT, OptT, std::vector<Tensor>> group_lora_bwd(const std::vector<Ten
 }
 
 // ------------------------------------------------------------------ the fused MLP
+// A weight's codes have as many columns as the product sums over: the adapters of a layer may fit where its base weight
+// does not, and the kernels would read past it.
+void check_cols(const char* what, const Tensor& w, int64_t k) {
+  TORCH_CHECK(w.dim() == 2 && w.size(1) == k, what, " of ", w.sizes(), ", a product over ", k, " columns");
+}
+
 // Every bf16 form of the step's LoRA weights (fused_mlp._prep): S, ST, bg, bu, bgT, buT, ad, adT, bd, bdT.
 std::vector<Tensor> mlp_forms(const std::array<Tensor, 6>& w, int64_t stream) {
   gpu(w[0], "mxfp8_lora_prep");
@@ -255,8 +269,10 @@ std::tuple<Tensor, Tensor, Tensor> mlp_forward(const Tensor& x, const Tensor& S,
                                                const Tensor& ad, const Tensor& bd, const Tensor& wf, const Tensor& wfs,
                                                const Tensor& wd, const Tensor& wds, double s_g, double s_u, double s_d,
                                                int64_t fold_sum, int64_t stream) {
-  gpu(x, "mxfp8_gemm_swiglu_fwd");
   const int64_t T = x.size(0), K = x.size(1), R = ad.size(0), N = ad.size(1);
+  check_cols("mlp_forward: gate|up weight", wf, K);
+  check_cols("mlp_forward: down weight", wd, N);
+  gpu(x, "mxfp8_gemm_swiglu_fwd");
   Tensor xs = empty({T, 2 * R}, kBF, x), gu = empty({ft_rows(T), 2 * N}, kBF, x), y;
   const int64_t parts = 2 * N / 128;
   const bool fold = R == 16 && T * R <= fold_sum;
@@ -299,8 +315,9 @@ std::tuple<Tensor, Tensor, Tensor> mlp_forward(const Tensor& x, const Tensor& S,
 // The same without the output (a checkpoint's recompute): (xs, gu).
 std::tuple<Tensor, Tensor> mlp_graph(const Tensor& x, const Tensor& S, const Tensor& w, const Tensor& ws, int64_t N,
                                      int64_t stream) {
-  gpu(x, "mxfp8_gemm_nt");
   const int64_t T = x.size(0), K = x.size(1), rp = S.size(0);
+  check_cols("mlp_graph: gate|up weight", w, K);
+  gpu(x, "mxfp8_gemm_nt");
   Tensor xs = empty({T, rp}, kBF, x), gu = empty({ft_rows(T), 2 * N}, kBF, x);
   Arena a;
   const int64_t q = a.take(tiled_rows(T) * K), s = a.take(scale_numel(T, K));
@@ -320,10 +337,12 @@ std::tuple<OptT, Tensor, Tensor, Tensor, Tensor, Tensor> mlp_backward(
     const Tensor& dy, const Tensor& x, const Tensor& xs, const Tensor& gu, const std::vector<Tensor>& f, const Tensor& wt,
     const Tensor& wts, const Tensor& wx, const Tensor& wxs, double s_g, double s_u, double s_d, int64_t SB, int64_t CG,
     bool wide, bool need_x, bool fp32_a, bool fp32_bd, int64_t stream) {
-  gpu(dy, "mxfp8_mlp_bwd");
   TORCH_CHECK(f.size() == 10, "mlp_backward: ten weight forms");
   const Tensor &ST = f[1], &bg = f[2], &bu = f[3], &bgT = f[4], &buT = f[5], &ad = f[6], &adT = f[7], &bdT = f[9];
   const int64_t T = dy.size(0), K = x.size(1), R = ad.size(0), N = ad.size(1), tpad = cdiv(T, 128) * 128;
+  check_cols("mlp_backward: down weight", wt, dy.size(1));
+  check_cols("mlp_backward: gate|up weight", wx, 2 * N);
+  gpu(dy, "mxfp8_mlp_bwd");
   const int64_t nsb = cdiv(tpad, SB), n_dxa = N / (wide ? 256 : 128), chunks = mxfp8_lora_tn_chunks(T, K);
   // a: until the finish, the codes of dy (read by the dh GEMM) under the partials (written after it); m: dhm; b: the
   // codes of dg | du; c: the finish's results; d: the token reductions' partials, made once a is dropped
