@@ -20,17 +20,46 @@ def _operands(M, N, K, gpu):
     return g, mxfp8.mx_quant_tiled(a), mxfp8.mx_quant_tiled(b), b
 
 
-# edges of 64, 128 and 256 rows; N that is and is not a multiple of 256; an odd count of 128-wide K tiles
-@pytest.mark.parametrize("M,N,K", [
-    (1, 128, 128), (63, 256, 384), (64, 1024, 1024), (65, 384, 640), (129, 2048, 1152),    # 64 x 64
-    (1000, 2048, 1024), (961, 1920, 1408),                                                 # 64 x 128
-    (129, 12288, 256), (1500, 2048, 2048), (1921, 1920, 1152),                             # 128 x 128
-    (321, 12288, 384), (1025, 12288, 128),                                                 # 256 x 128
-    (5000, 2048, 2048), (4353, 2304, 1280),                                                # 256 x 256
-    # 256 x 128, the rows past the last whole round of tiles in 64 x 128 or 128 x 128 tiles: 1 to 704 such rows, after
-    # one workgroup per CU and after two
-    (1281, 12288, 384), (1407, 6144, 256), (3840 + 257, 6272, 640), (8896, 2048, 1152), (5377, 1920, 2048),  # 64 x 128
-    (2753, 12288, 128), (3073, 6272, 640), (9217, 2048, 1152)])                                              # 128 x 128
+# (the shape, the shape of the last rows or None) that a GPU of 256 CUs takes -> sizes: edges of 64, 128 and 256 rows; N
+# that is and is not a multiple of 256; an odd count of 128-wide K tiles.  test_gemm_shape_rule.py holds the sizes to
+# their shapes.
+SIZES = {
+    ("64x64", None): [(1, 128, 128), (63, 256, 384), (64, 1024, 1024), (65, 384, 640), (129, 2048, 1152)],
+    ("64x128", None): [(1000, 2048, 1024), (961, 1920, 1408)],
+    ("128x128", None): [(129, 12288, 256), (1500, 2048, 2048), (1921, 1920, 1152)],
+    ("256x128", None): [(321, 12288, 384), (1025, 12288, 128)],
+    ("256x256", None): [(770, 12288, 3072), (2561, 4096, 3072), (5131, 2048, 3072)],
+    # the rows past the last whole round of tiles: 1 to 1024 such rows, after one workgroup per CU and after two
+    ("256x128", "64x128"): [(1281, 12288, 384), (1407, 6144, 256), (3840 + 257, 6272, 640), (8896, 2048, 1152),
+                            (5377, 1920, 2048), (5000, 2048, 2048), (4353, 2304, 1280)],
+    ("256x128", "128x128"): [(2753, 12288, 128), (3073, 6272, 640), (9217, 2048, 1152)],
+}
+# the same for mxfp8_gemm_nt_sum and mxfp8_gemm_nt_tn (which lose their folded work's share in the 8-wave shape)
+FOLDED = {
+    ("64x64", None): [(65, 384, 640)],
+    ("64x128", None): [(961, 1920, 1408)],
+    ("128x128", None): [(1921, 1920, 1152)],
+    ("256x128", None): [(321, 12288, 384)],
+    ("256x256", None): [(10497, 12288, 3072)],
+    ("256x128", "64x128"): [(4097, 2048, 1152)],
+    ("256x128", "128x128"): [(9217, 2048, 1152)],
+}
+# the same for mxfp8_gemm_nt_seg: (M, output widths, K)
+SEGMENTS = {
+    ("64x64", None): [(40, (256, 128, 256), 256)],
+    ("64x128", None): [(700, (1024, 256, 256), 1024)],
+    ("128x128", None): [(1500, (1024, 256, 256), 1024)],
+    ("256x128", None): [(3073, (2048, 2048), 2048)],
+    ("256x128", "64x128"): [(5377, (1280, 512, 128), 2048)],
+    ("256x128", "128x128"): [(4300, (4096, 1920, 128, 128), 640)],
+}
+
+
+def _sizes(table):
+    return [size for sizes in table.values() for size in sizes]
+
+
+@pytest.mark.parametrize("M,N,K", _sizes(SIZES))
 @pytest.mark.parametrize("rank", [0, 16, 48])
 def test_every_shape_gives_the_same_bits(M, N, K, rank, gpu):
     g, (qa, sa), (qb, sb), b = _operands(M, N, K, gpu)
@@ -54,20 +83,20 @@ def test_every_shape_gives_the_same_bits(M, N, K, rank, gpu):
     assert torch.equal(ft[0].view(torch.int16), ft[1].view(torch.int16))
 
 
-@pytest.mark.parametrize("M,N,K", [(65, 384, 640), (961, 1920, 1408), (1921, 1920, 1152), (20501, 2048, 12288),
-                                   (4097, 2048, 1152), (9217, 2048, 1152)])
+@pytest.mark.parametrize("M,N,K", _sizes(FOLDED) + [(20501, 2048, 12288)])
 def test_folded_launches_in_every_shape(M, N, K, gpu):
     """mxfp8_gemm_nt_sum and mxfp8_gemm_nt_tn against the separate calls, in the shapes that carry the folded work and
-    in the 8-wave one, which launches it apart: bit-identical."""
+    in the 8-wave one, which launches it apart: bit-identical.  wait_limit 0: every tile sums its own rows of P."""
     g, (qa, sa), (qb, sb), _ = _operands(M, N, K, gpu)
     part = torch.randn(5, M, 16, device=gpu, generator=g)
     Q = (torch.randn(N, 32, device=gpu, generator=g) * 0.1).to(torch.bfloat16)
     P = torch.empty(M, 16, dtype=torch.bfloat16, device=gpu)
     _native.sum_parts(part, 5, M * 16, P)
     want = mxfp8.mx_mm(qa, sa, qb, sb, lora=(P, Q[:, :16]), alpha=0.5, layout=3, m=M)
-    P2 = torch.empty_like(P)
-    got = mxfp8.mx_mm_sum(qa, sa, qb, sb, part, P2, Q[:, :16], 0.5, 3, M)
-    assert torch.equal(P, P2) and torch.equal(got.view(torch.int16), want.view(torch.int16))
+    for wait_limit in (-1, 0):
+        P2 = torch.full_like(P, float("nan"))
+        got = mxfp8.mx_mm_sum(qa, sa, qb, sb, part, P2, Q[:, :16], 0.5, 3, M, wait_limit=wait_limit)
+        assert torch.equal(P, P2) and torch.equal(got.view(torch.int16), want.view(torch.int16)), wait_limit
     x = torch.randn(M, 256, device=gpu, generator=g).to(torch.bfloat16)
     P3 = torch.randn(M, 32, device=gpu, generator=g).to(torch.bfloat16)
     outs = [torch.empty(32, 256, dtype=torch.bfloat16, device=gpu) for _ in range(2)]
@@ -76,6 +105,37 @@ def test_folded_launches_in_every_shape(M, N, K, gpu):
     _native.lora_tn_batch([(x, P3, outs[0], 1.0, False)], scratch)
     got = mxfp8.mx_mm_tn(qa, sa, qb, sb, (P3, Q), 1.0, 3, M, [(x, P3, outs[1], 1.0, False)], scratch)
     assert torch.equal(outs[0], outs[1]) and torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("M,widths,K", _sizes(SEGMENTS))
+@pytest.mark.parametrize("rank,window", [(0, False), (48, False), (16, True)])
+def test_separate_outputs_in_every_shape(M, widths, K, rank, window, gpu):
+    """mxfp8_gemm_nt_seg against one GEMM per output in the 8-wave shape: bit-identical.  window: each output adds the
+    rank-16 product over columns of its own (the others hold NaN), else all over the same 48."""
+    N = sum(widths)
+    g, (qa, sa), (qb, sb), _ = _operands(M, N, K, gpu)
+    P = (torch.randn(M, 64, device=gpu, generator=g) * 0.1).to(torch.bfloat16)
+    Q = (torch.randn(N, 64, device=gpu, generator=g) * 0.1).to(torch.bfloat16)
+    cols = [16 * k for k in range(len(widths))] if window else [0] * len(widths)
+    per_tile_row, c0, want = K // 128 * 512, 0, []
+    for n, col in zip(widths, cols):
+        lora = (P[:, col:col + rank], Q[c0:c0 + n, col:col + rank]) if rank else None
+        out = torch.full((M, n), float("nan"), dtype=torch.bfloat16, device=gpu)
+        scales = sb[c0 // 128 * per_tile_row:(c0 + n) // 128 * per_tile_row]
+        _native.gemm_nt(qa, sa, K, qb[c0:c0 + n], scales, K, M, n, K, out, lora=lora, alpha=0.7, split=False,
+                        layout=3 | _native.GEMM_WIDE)
+        want.append(out)
+        if window:
+            keep = Q[c0:c0 + n, col:col + rank].clone()
+            Q[c0:c0 + n] = float("nan")
+            Q[c0:c0 + n, col:col + rank] = keep
+        c0 += n
+    outs = [torch.full((M, n), float("nan"), dtype=torch.bfloat16, device=gpu) for n in widths]
+    lora = (P if window else P[:, :rank], Q if window else Q[:, :rank]) if rank else None
+    kw = dict(lora_cols=cols, r=rank) if window else {}
+    mxfp8.mx_mm_seg(qa, sa, qb, sb, outs, lora=lora, alpha=0.7, layout=3, m=M, **kw)
+    for k, (a, b) in enumerate(zip(outs, want)):
+        assert torch.equal(a.view(torch.int16), b.view(torch.int16)), k
 
 
 @pytest.mark.parametrize("rank", [0, 16])

@@ -225,6 +225,16 @@ def scratch_f32(n, device):
     return buf
 
 
+GEMM_KINDS = ("plain", "sum", "tn", "seg")
+
+
+def gemm_shape(M, N, K, kind="plain", cus=256):
+    """(workgroup shape, shape of its last rows or None, their first row) of a GEMM of this size on a GPU of `cus` CUs:
+    kind "plain" (gemm_nt), "sum" (gemm_nt_sum), "tn" (mxfp8_gemm_nt_tn) or "seg" (gemm_nt_seg with two outputs or more).
+    Host code only; results do not depend on the shape."""
+    return host().gemm_shape(M, N, K, GEMM_KINDS.index(kind), cus)
+
+
 def gemm_nt(a, sa, lda, b, sb, ldb, M, N, K, c, lora=None, alpha=1.0, split=True, layout=0):
     """c[M, N] = bf16(A·Bᵀ) [+ alpha · P·Qᵀ with lora = (P [M, r], Q [N, r])].  layout bit 0 / 1: A / B codes
     MX-tiled; bit 2 (GEMM_WIDE): 8-wave 256 x 256 workgroups, whose tail tiles split along K through the cached

@@ -24,6 +24,7 @@
 #include <vector>
 
 #include "../../include/mxfp8_mlp.h"
+#include "gemm_shape.h"
 
 namespace py = pybind11;
 using at::Tensor;
@@ -143,6 +144,20 @@ std::vector<Tensor> gemm_seg(const Tensor& q, const Tensor& s, const Tensor& w, 
                          rcols.empty() ? nullptr : rcols.data(), (float)alpha, layout, stm(stream)),
        "mxfp8_gemm_nt_seg");
   return outs;
+}
+
+// The rule by which the library takes a GEMM's workgroup shape: (shape, shape of the rows from tail_row on, tail_row).
+std::tuple<std::string, std::optional<std::string>, int64_t> gemm_shape(int64_t M, int64_t N, int64_t K, int64_t kind,
+                                                                        int64_t cus) {
+  TORCH_CHECK(M > 0 && N > 0 && K > 0 && M < (1LL << 30) && N < (1LL << 30) && K < (1LL << 30) && N % 128 == 0 &&
+                  K % 128 == 0 && kind >= 0 && kind <= mxk::kGemmSeg && cus > 0 && cus < (1 << 20),
+              "gemm_shape: bad size or kind");
+  const auto name = [](mxk::ShapeId id) {
+    const auto& c = mxk::kCost[(int)id];
+    return std::to_string(c.bm) + "x" + std::to_string(c.bn);
+  };
+  const mxk::Pick p = mxk::pick_shape(M, N, K, (int)cus, (mxk::GemmKind)kind);
+  return {name(p.shape), p.tail_row ? std::optional<std::string>(name(p.tail)) : std::nullopt, p.tail_row};
 }
 
 using TnJob = std::tuple<Tensor, Tensor, Tensor, double, bool>;  // x, p, out, scale, transpose
@@ -423,6 +438,7 @@ PYBIND11_MODULE(_mxhost, m) {
   def("quant_tiled", &quant_tiled);
   def("quant_lora", &quant_lora);
   def("gemm", &gemm);
+  def("gemm_shape", &gemm_shape);
   def("gemm_seg", &gemm_seg);
   def("gemm_tn", &gemm_tn);
   def("res_lora", &res_lora);
