@@ -178,12 +178,6 @@ def quant_dual(x, q, s, qt, st):
     call("mxfp8_quant_dual", _p(x), R, C, x.stride(0), _p(q), _p(s), _p(qt), _p(st), like=x)
 
 
-def quant_tiled(x, q, s):
-    """x [R, C] bf16 -> codes in the MX-tiled layout into q (ceil(R/16)*16 * C bytes) and blocked scales."""
-    R, C = x.shape
-    call("mxfp8_quant_tiled", _p(x), R, C, x.stride(0), _p(q), _p(s), like=x)
-
-
 def tile_codes(q, rows, cols, out):
     """Row-major codes (row stride q.stride(0)) -> the MX-tiled layout into out."""
     call("mxfp8_tile_codes", _p(q), rows, cols, q.stride(0), _p(out), like=out)
@@ -354,13 +348,6 @@ def quant_lora_tp(x, q, s, w, out, tx, tout, scale=1.0, outT=None):
          _p(outT), -(-T // 128) * 128, _p(tx), tx.stride(0), tx.shape[1], _p(tout), like=x)
 
 
-def res_lora(x, y, xa, b, out, scale):
-    """out = bf16(x + bf16(y + scale · xa · bᵀ)); x, y, out [T, N], xa [T, r] (row stride any), b [N, r]."""
-    T, N = x.shape
-    call("mxfp8_res_lora", _p(x), _p(y), _p(xa), xa.stride(0), _p(b), T, N, b.shape[1], float(scale), _p(out),
-         like=x)
-
-
 def swiglu(g, u, h):
     """h = bf16(silu(g) · u) elementwise (bf16, contiguous, numel % 8 == 0)."""
     call("mxfp8_swiglu", _p(g), _p(u), g.numel(), _p(h), like=g)
@@ -419,18 +406,6 @@ def _tn_table(jobs, part, chunks):
     table = [LoraTnJob(_p(x), x.stride(0), _p(p), p.shape[1], float(sc), int(tr), int(out.dtype == torch.float32),
                        _p(out)) for x, p, out, sc, tr in jobs]
     return (LoraTnJob * len(table))(*table), len(table), T, K, chunks
-
-
-def gemm_nt_tn(a, sa, lda, b, sb, ldb, M, N, K, c, lora, jobs, part, alpha=1.0, layout=0, chunks=None):
-    """gemm_nt (rank-16, 32 or 48 lora = (P, Q), 4-wave shape) and lora_tn_batch(jobs, part, chunks) in one launch,
-    plus the batch's sums (include/mxfp8_mlp.h, mxfp8_gemm_nt_tn): the token reductions fill the GEMM's idle tail
-    slots."""
-    p, q = lora
-    arr, n, T, Kt, chunks = _tn_table(jobs, part, chunks)
-    _gpu(c, "mxfp8_gemm_nt_tn")
-    call("mxfp8_gemm_nt_tn", _p(a), _p(sa), lda, _p(b), _p(sb), ldb, M, N, K, _p(c), c.stride(0), _p(p),
-         p.stride(0), _p(q), q.stride(0), p.shape[1], float(alpha), layout, ctypes.cast(arr, _ptr), n, T, Kt, chunks,
-         _p(part), like=c)
 
 
 class LoraBwdJob(ctypes.Structure):

@@ -147,7 +147,8 @@ def lora_bwd_batch(dys, xas, Bs, scales, dxa_outs, q=None, s=None, col_tile_offs
     """lora_bwd of the layers of a group (one shared T and rank r) in one launch and one launch of their partial
     sums (mxfp8_lora_bwd_batch): every dy streams at once, with one row chunking for all.  Same arguments per
     layer as lora_bwd; returns the layers' dB (fp32).  d(xa) is the same bits as lora_bwd's; dB adds its row
-    chunks in another grouping (fp32 rounding)."""
+    chunks in another grouping (fp32 rounding).  The grouped backward makes this call through the host module, with
+    MX-tiled codes (_native.host().group_lora_bwd); here the codes are row-major."""
     T, R = dys[0].shape[0], xas[0].shape[1]
     assert 1 <= len(dys) <= _native.LORA_BWD_MAX_JOBS and R in (16, 32) and T > 0, (len(dys), R, T)
     if q is not None:
