@@ -447,7 +447,7 @@ def _traffic_summary(cfg, fetch_dir, write_dir, cmd_fetch, cmd_write):
         for (_, name, grid), v in vals.items():
             if "gemm_kernel" not in name:
                 continue
-            m = re.search(r"(\w*gemm_kernel<[^>]*>)", name)
+            m = re.search(r"(\w*gemm_kernel<[^>]*>)", _gemm_name(name))
             g.setdefault((m.group(1) if m else name[:60], grid), []).append(v)
         return {k: (sum(v) / len(v), len(v)) for k, v in g.items()}
 
@@ -510,7 +510,7 @@ _TABLE_CAPTIONS = {
         "T = 10752 tokens, r = 16. The run times `lora_bwd` at dy [T, 2048] (grid y = 16) and [T, 6144] (y = 48) and "
         "`res_lora` at [T, 2048] (50 calls each), then 13 steps (3 warmup + 10) of the attention-projection step "
         "(q|k|v 2048/512/512 grouped, o_proj 2048 -> 2048 deferred into `residual_add`, forward + backward; the dx "
-        "GEMMs, `gemm_kernel<48, 1, 0>` and `<16, 1, 0>` with 928 workgroups, run the dA reductions in their launch), "
+        "GEMMs, `gemm_kernel<48, 256x128, 0>` and `<16, 256x128, 0>` with 928 workgroups, run the dA reductions in their launch), "
         "3 more on a side stream and 13 replays of the step captured into a HIP graph, then the "
         "SwiGLU kernels alone on [T, 6144] and 13 steps of the unfused MLP (`shared_prefix._mlp` with the fused MLP "
         "off: gate and up as one `group_linear`, the SwiGLU kernels, down as a `group_linear`; gate/up/down are not "
@@ -538,7 +538,7 @@ def _kernel_table(name, d, cmd, min_calls=6):
                     m = re.search(r"_MT(\d+x\d+x\d+)_", kname)
                     key = f"hipBLASLt GEMM (MT{m.group(1) if m else '?'})"
                 else:
-                    key = re.sub(r"\(anonymous namespace\)::", "", kname).split("(")[0].replace("void ", "")
+                    key = re.sub(r"\(anonymous namespace\)::", "", _gemm_name(kname)).split("(")[0].replace("void ", "")
                 wg = max(int(r.get("Workgroup_Size_X") or 1), 1)
                 grid = f"{int(r['Grid_Size_X']) // wg} x {r['Grid_Size_Y']}"
                 agg.setdefault((key, grid), []).append((int(r["End_Timestamp"]) - int(r["Start_Timestamp"])) / 1e3)
@@ -559,11 +559,31 @@ def _md(text):
     return text.replace("|", "\\|")
 
 
+_SHAPE_RE = r"(?:\(anonymous namespace\)::)?Shape<([\d, ]+)>"
+
+
+def _tile(args):
+    """The rows x columns of a GEMM workgroup's tile, from its Shape's template arguments (blocks of 32 a wave and waves
+    along both axes, csrc/mx_gemm.hip)."""
+    mb, nb, wm, wn = [int(a) for a in args.split(",")[:4]]
+    return f"{32 * mb * wm}x{32 * nb * wn}"
+
+
+def _gemm_name(name):
+    """A kernel name with an MX GEMM's workgroup shapes as tiles: gemm_kernel<epilogue rank, tile[ + tile of the last
+    rows], epilogue>; other names as they are."""
+    def short(m):
+        a, b = _tile(m.group(2)), _tile(m.group(4))
+        return f"gemm_kernel<{m.group(1)}, {a}{'' if a == b else ' + ' + b}, {m.group(3)}>"
+    return re.sub(r"gemm_kernel<(\d+), " + _SHAPE_RE + r", (\d+), " + _SHAPE_RE + r" ?>", short, name)
+
+
 def _kernel_key(name, grid):
     """A short kernel name: the template head of the demangled name, and for the MX GEMM the MLP shape its grid
     and epilogue rank identify at configuration 3 (4032 / 2016 / 672 workgroups of 256 threads; the dx GEMM with
     the backward's token reductions folded into its launch has 672 + 512, the down GEMM with the xS_down sum
     168 + 672)."""
+    name = _gemm_name(name)
     m = re.search(r"(\w+_kernel)(<[^>]*>)?", name)
     k = (m.group(1) + (m.group(2) or "")) if m else name[:48]
     if m and m.group(1) == "gemm_kernel":
@@ -724,12 +744,12 @@ def _trace_summary(name, d, steps, cmd, layers=1):
                 srows = list(csv.DictReader(fh))
             f.write("\nrocprofv3 --stats of the same run (every dispatch of the process by kernel name, the gating "
                     "forward and the warmup steps included; in the MLP step each MX GEMM shape has its own template "
-                    "arguments: <16, 1, 1> gate|up with the SwiGLU epilogue, <16, 1, 0> down (with the xS_down "
-                    "sum in its launch by default), <0, 1, 0> dh, <32, 1, 0> dx (with the token reductions in its "
-                    "launch by default)):\n\n| kernel | calls | average us | min us | max us | % |\n"
+                    "arguments, epilogue rank, tile and epilogue: 16 and 1 gate|up with the SwiGLU epilogue, 16 and 0 down "
+                    "(with the xS_down sum in its launch where that is 4 waves), 0 and 0 dh, 32 and 0 dx (with the "
+                    "token reductions in its launch likewise)):\n\n| kernel | calls | average us | min us | max us | % |\n"
                     "|---|---|---|---|---|---|\n")
             for r in srows[:16]:
-                m = re.search(r"(\w+_kernel)(<[^>]*>)?", r["Name"])
+                m = re.search(r"(\w+_kernel)(<[^>]*>)?", _gemm_name(r["Name"]))
                 kn = (m.group(1) + (m.group(2) or "")) if m else r["Name"][:48]
                 f.write(f"| {kn} | {r['Calls']} | {float(r['AverageNs']) / 1e3:.1f} | "
                         f"{float(r['MinNs']) / 1e3:.1f} | {float(r['MaxNs']) / 1e3:.1f} | "

@@ -87,6 +87,21 @@ def test_gemm_shape_names(name, grid, want):
     assert bench._kernel_key(name, grid).endswith(want)
 
 
+_TALL, _LOW, _WIDE = ("(anonymous namespace)::Shape<%s>" % a for a in ("2, 4, 4, 1, 1, 3", "1, 2, 2, 2, 2, 3",
+                                                                       "2, 4, 4, 2, 1, 4"))
+
+
+@pytest.mark.parametrize("args,grid,want", [
+    (f"16, {_TALL}, 1, {_TALL}", 4032, "gemm_kernel<16, 256x128, 1> gate|up + SwiGLU epilogue"),
+    (f"32, {_TALL}, 0, {_TALL}", 1184, "gemm_kernel<32, 256x128, 0> dx + token reductions"),
+    (f"16, {_TALL}, 0, {_TALL}", 840, "gemm_kernel<16, 256x128, 0> down + xS_down sum"),
+    (f"0, {_WIDE}, 0, {_WIDE}", 8896, "gemm_kernel<0, 256x256, 0> dh"),
+    (f"32, {_TALL}, 0, {_LOW}", 900, "gemm_kernel<32, 256x128 + 64x128, 0> dx")])
+def test_gemm_names_with_their_tiles(args, grid, want):
+    name = f"void (anonymous namespace)::gemm_kernel<{args} >(unsigned char const*, long, int)"
+    assert bench._kernel_key(name, str(grid * 256)) == want
+
+
 def test_more_than_one_gpu_is_refused():
     r = subprocess.run([sys.executable, os.path.join(ROOT, "bench.py"), "--gpus", "2"], capture_output=True,
                        text=True, timeout=120)
