@@ -15,9 +15,14 @@ enum class ShapeId { kTall, kWide, kMid, kLow, kSmall };
 // Estimated us of a launch in one shape, from the size alone: with w = tiles per CU and rounds = ceil(w),
 //   K steps * (step * rounds + fill * w + (one round: lone) + late * max(0, w - 8)) + round * rounds + base.
 // A round costs its K steps' serial part (barrier, fragment reads) whether or not it fills the chip (`step`), the
-// rest grows with the tiles (`fill`); `late` is what long launches lose to the L2 and the clock.  Least squares
-// over 13 shapes (N 1024-12288, K 1024-12288) at 20 values of M from 64 to 142336, on one MI355X: relative error
-// 3-4% (standard deviation); over those sizes the shape it picks takes 0.2% longer than the fastest one on average.
+// rest grows with the tiles (`fill`); `late` is what long launches lose to the L2 and the clock.  Least squares over 13
+// shapes (N 1024-12288, K 1024-12288) at 20 values of M from 64 to 142336, on one MI355X, with a residual of 3-4%
+// (standard deviation); over those sizes the shape it picks takes 0.2% longer than the fastest one on average.  It ranks
+// shapes and is no prediction of a launch inside a pass: there, over the 17 plain GEMMs of the timed workloads, a launch
+// takes 0.91 to 1.38 times the estimate: long K and wide N within 10%, (M, N, K) = (4096, 2048, 2048) 24.5 us for 17.8,
+// (10752, 2048, 2048) 50.8 for 44.3, (10752, 3072, 2048) 71 for 61, (4096, 1024, 3584) 23.6 for 18.9 in Mid, (256, 1024,
+// 3584) 11.2 for 8.6 in Small.  Operands from memory are not the cause: the same launch over and over on the same
+// operands takes 23.4, 51, 72, 21.6 and 9.1 us.
 struct ShapeCost {
   int bm, bn;
   float step, fill, lone, late, round, base;

@@ -359,58 +359,61 @@ std::tuple<OptT, Tensor, Tensor, Tensor, Tensor, Tensor> mlp_backward(
   check_cols("mlp_backward: gate|up weight", wx, 2 * N);
   gpu(dy, "mxfp8_mlp_bwd");
   const int64_t nsb = cdiv(tpad, SB), n_dxa = N / (wide ? 256 : 128), chunks = mxfp8_lora_tn_chunks(T, K);
-  // a: until the finish, the codes of dy (read by the dh GEMM) under the partials (written after it); m: dhm; b: the
-  // codes of dg | du; c: the finish's results; d: the token reductions' partials, made once a is dropped
-  Arena a, m, b, c, d;
-  const int64_t dxd = a.take(T * R * 2), dxdT = a.take(R * tpad * 2), xsT = a.take(2 * R * tpad * 2);
-  const int64_t under = a.total, qd = a.take(tiled_rows(T) * dy.size(1)), sd = a.take(scale_numel(T, dy.size(1)));
-  const int64_t codes_end = a.total;
-  a.total = under;
+  // m: dhm, dropped after the backward kernel; a, dropped after the finish: the codes of dy (read by the dh GEMM) under the
+  // partials (written after it); b: the codes of dg | du, and dxd and the transposed operands (read by the backward
+  // kernel) under the finish's results; c: the token reductions' partials, made when a is gone
+  Arena m, a, b, c;
+  const int64_t dhm = m.take(ft_rows(T) * N * 2);
+  const int64_t qd = a.take(tiled_rows(T) * dy.size(1)), sd = a.take(scale_numel(T, dy.size(1))), end_a = a.total;
+  a.total = 0;
   const int64_t dxa_p = a.take(n_dxa * T * 3 * R * 4), dbg_p = a.take(nsb * N * R * 4), dbu_p = a.take(nsb * N * R * 4),
                 dad_p = a.take(nsb * R * N * 4);
-  a.total = std::max(a.total, codes_end);
-  const int64_t dhm = m.take(ft_rows(T) * N * 2);
-  const int64_t qg = need_x ? b.take(tiled_rows(T) * 2 * N) : 0, sg = need_x ? b.take(scale_numel(T, 2 * N)) : 0;
-  const int64_t dxa = c.take(T * 2 * R * 2), xsd = c.take(T * R * 2), part = d.take(chunks * 3 * R * K * 4);
+  a.total = std::max(a.total, end_a);
+  const int64_t qg = need_x ? b.take(tiled_rows(T) * 2 * N) : 0, sg = need_x ? b.take(scale_numel(T, 2 * N)) : 0,
+                under_b = b.total;
+  const int64_t dxd = b.take(T * R * 2), dxdT = b.take(R * tpad * 2), xsT = b.take(2 * R * tpad * 2), end_b = b.total;
+  b.total = under_b;
+  const int64_t dxa = b.take(T * 2 * R * 2), xsd = b.take(T * R * 2);
+  b.total = std::max(b.total, end_b);
+  const int64_t part = c.take(chunks * 3 * R * K * 4);
   a.make(dy);
   m.make(dy);
+  b.make(dy);
   void* const st = stm(stream);
-  ok(mxfp8_quant_lora_tp(ptr(dy), T, dy.size(1), dy.stride(0), a.at(qd), a.at(sd), ptr(bdT), R, (float)s_d, a.at(dxd),
-                         a.at(dxdT), tpad, ptr(xs), xs.stride(0), 2 * R, a.at(xsT), st),
+  ok(mxfp8_quant_lora_tp(ptr(dy), T, dy.size(1), dy.stride(0), a.at(qd), a.at(sd), ptr(bdT), R, (float)s_d, b.at(dxd),
+                         b.at(dxdT), tpad, ptr(xs), xs.stride(0), 2 * R, b.at(xsT), st),
      "mxfp8_quant_lora_tp");
   const int64_t tt = MXFP8_GEMM_A_TILED | MXFP8_GEMM_B_TILED;
   ok(mxfp8_gemm_nt(a.at(qd), a.at(sd), dy.size(1), ptr(wt), ptr(wts), dy.size(1), T, N, dy.size(1), m.at(dhm), N, nullptr,
                    0, nullptr, 0, 0, 1.f, tt | MXFP8_GEMM_C_FT | MXFP8_GEMM_B_PI, nullptr, 0, st),
      "mxfp8_gemm_nt");
-  if (need_x) b.make(dy);
-  ok(mxfp8_mlp_bwd(ptr(gu), ptr(xs), a.at(xsT), m.at(dhm), a.at(dxd), a.at(dxdT), ptr(bg), ptr(bu), ptr(bgT), ptr(buT),
+  ok(mxfp8_mlp_bwd(ptr(gu), ptr(xs), b.at(xsT), m.at(dhm), b.at(dxd), b.at(dxdT), ptr(bg), ptr(bu), ptr(bgT), ptr(buT),
                    ptr(ad), ptr(adT), T, N, R, (float)s_g, (float)s_u, SB, CG, need_x ? b.at(qg) : nullptr,
                    need_x ? b.at(sg) : nullptr, a.f(dxa_p), a.f(dbg_p), a.f(dbu_p), a.f(dad_p), nullptr,
                    1 | 2 | (wide ? 4 : 0), st),
      "mxfp8_mlp_bwd");
   m.drop();
-  c.make(dy);
-  Tensor dA = empty({2 * R, K}, fp32_a ? kF32 : kBF, dy), dBg = empty({N, R}, kF32, dy), dBu = empty({N, R}, kF32, dy),
-         dAd = empty({R, N}, kF32, dy), dBd = empty({K, R}, fp32_bd ? kF32 : kBF, dy);
+  Tensor dBg = empty({N, R}, kF32, dy), dBu = empty({N, R}, kF32, dy), dAd = empty({R, N}, kF32, dy);
   ok(mxfp8_mlp_bwd_finish(a.f(dxa_p), a.f(dbg_p), a.f(dbu_p), a.f(dad_p), n_dxa, nsb, T, N, R, (float)s_g, (float)s_u,
-                          c.at(dxa), c.at(xsd), fptr(dBg), fptr(dBu), fptr(dAd), st),
+                          b.at(dxa), b.at(xsd), fptr(dBg), fptr(dBu), fptr(dAd), st),
      "mxfp8_mlp_bwd_finish");
   a.drop();
-  d.make(dy);
-  const mxfp8_lora_tn_job jobs[2] = {{ptr(dy), dy.stride(0), c.at(xsd), R, (float)s_d, 1, fp32_bd, ptr(dBd)},
-                                     {ptr(x), x.stride(0), c.at(dxa), 2 * R, 1.f, 0, fp32_a, ptr(dA)}};
+  c.make(dy);
+  Tensor dA = empty({2 * R, K}, fp32_a ? kF32 : kBF, dy), dBd = empty({K, R}, fp32_bd ? kF32 : kBF, dy);
+  const mxfp8_lora_tn_job jobs[2] = {{ptr(dy), dy.stride(0), b.at(xsd), R, (float)s_d, 1, fp32_bd, ptr(dBd)},
+                                     {ptr(x), x.stride(0), b.at(dxa), 2 * R, 1.f, 0, fp32_a, ptr(dA)}};
   const bool fold = need_x && R == 16;
-  if (!fold) ok(mxfp8_lora_tn_batch(jobs, 2, T, K, chunks, d.f(part), st), "mxfp8_lora_tn_batch");
+  if (!fold) ok(mxfp8_lora_tn_batch(jobs, 2, T, K, chunks, c.f(part), st), "mxfp8_lora_tn_batch");
   OptT dx;
   if (need_x) {
     dx = empty({T, K}, kBF, dy);
     const int64_t lay = tt | MXFP8_GEMM_B_PI;
     if (fold)
-      ok(mxfp8_gemm_nt_tn(b.at(qg), b.at(sg), 2 * N, ptr(wx), ptr(wxs), 2 * N, T, K, 2 * N, ptr(dx), K, c.at(dxa), 2 * R,
-                          ptr(ST), ST.stride(0), 2 * R, 1.f, lay, jobs, 2, T, K, chunks, d.f(part), st),
+      ok(mxfp8_gemm_nt_tn(b.at(qg), b.at(sg), 2 * N, ptr(wx), ptr(wxs), 2 * N, T, K, 2 * N, ptr(dx), K, b.at(dxa), 2 * R,
+                          ptr(ST), ST.stride(0), 2 * R, 1.f, lay, jobs, 2, T, K, chunks, c.f(part), st),
          "mxfp8_gemm_nt_tn");
     else
-      ok(mxfp8_gemm_nt(b.at(qg), b.at(sg), 2 * N, ptr(wx), ptr(wxs), 2 * N, T, K, 2 * N, ptr(dx), K, c.at(dxa), 2 * R,
+      ok(mxfp8_gemm_nt(b.at(qg), b.at(sg), 2 * N, ptr(wx), ptr(wxs), 2 * N, T, K, 2 * N, ptr(dx), K, b.at(dxa), 2 * R,
                        ptr(ST), ST.stride(0), 2 * R, 1.f, lay, nullptr, 0, st),
          "mxfp8_gemm_nt");
   }

@@ -210,9 +210,10 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(kFwdWavesPe
 // (151.9-154.7 against 148.9-152.4 us at configuration 3, three alternating pairs on one box, bit-identical).
 // The products are written, summed and stored in 16-byte pieces (rows of 3r + 4 floats: the 16 lanes that an LDS access
 // serves at a time start in different banks); kMain fixes the FT and MX-tiled layouts, the ones of the fused path, at
-// compile time (with r = 32 it spills more and was slower).  A row block is bound by its serial chain (VALU about 60%
-// of it, its barrier, these LDS passes), not by memory: us with 4-byte pieces -> 16-byte pieces -> kMain, r = 16,
-// N = 6144: T = 2048 36.8 -> 35.7 -> 35.2, T = 10752 144 -> 138 -> 136; r = 32, T = 10752 195 -> 183.
+// compile time (with r = 32 it spills more and was slower; the form that runs there spills 58 registers, 200 bytes a
+// lane).  A row block is bound by its serial chain (VALU about 60% of it, its barrier, these LDS passes), not by memory:
+// us with 4-byte pieces -> 16-byte pieces -> kMain, r = 16, N = 6144: T = 2048 36.8 -> 35.7 -> 35.2, T = 10752 144 ->
+// 138 -> 136; r = 32, T = 10752 195 -> 183.
 // gu is read once here, with non-temporal loads, so it does not push dhm (written by the GEMM just before) and
 // the MX(dg | du) codes out of the last-level cache (with the gate|up epilogue's non-temporal gu stores, MX_NT_GU
 // in mx_gemm.hip: 10-17 us per configuration-3 step faster over five A/B pairs on one box).

@@ -27,10 +27,12 @@
 // L2.  A Tall launch whose last tiles would run alone on their CUs gives those rows to Mid or Low tiles in the same
 // launch (its tail).  pick_shape (gemm_shape.h) chooses.
 //
-// What bounds it (rocprofv3 counters): with this order the matrix pipe is busy 71% (Tall) to 74% (Wide) of a long
-// launch at 1.72 and 1.52 GHz, so the power limit holds it; products of a step in serpentine order, which keep one
-// operand from each to the next, gained 0.3-0.8% there.  Before, the CU's vector-memory path that carries the operand
-// DMA held it (TA / TD busy 65-89%) at a matrix pipe busy ~48%.  An L2 prefetch ahead of the ring made it slower.
+// What bounds it (rocprofv3 counters, profiles/mlp_c4_counters.md and mlp_c3_counters.md; share of the matrix pipe's cycles
+// at the sustained clock, 2.4 GHz unloaded): at T = 142336 dx 80% at 1.63 GHz, down 74% at 1.65, dh 63% at 1.86 (Wide),
+// gate|up 61% at 1.71 (Tall); at T = 10752 50-61% at 1.92-2.11 GHz (Tall).  So the clock that the power limit leaves takes
+// a quarter to a third of the long launches, and the waves' waits the rest; the short launches lose more to their last
+// round of tiles and epilogues.  Products of a step in serpentine order, which keep one operand from each to the next,
+// gained 0.3-0.8% on the long ones.  An L2 prefetch ahead of the ring made it slower.
 //
 // Operand layouts: row-major codes (row stride lda / ldb), or the MX-tiled layout (tiled_offset in
 // mx_device.h) in which each 16-row x 64-code slice is one contiguous 1 KB block in LDS order.  The GEMM is
@@ -107,9 +109,11 @@ struct Shape {
   static constexpr int kDma = kKS * (kSA + kSB) + kSS;
   static constexpr int64_t kPartBytes = (int64_t)kBM * kBN * 4;  // fp32 partial tile
 };
+// Workgroups per CU: the ring's LDS bounds Tall, Low and Small at two and Wide at one; Mid's would hold three, as would its
+// 143-154 registers, but gemm_kernel is compiled for two waves per SIMD in every shape (amdgpu_waves_per_eu).
 using Tall = Shape<2, 4, 4, 1, 1, 3>;   // 256 x 128, 4 waves, ring 78 KB: two workgroups per CU
 using Wide = Shape<2, 4, 4, 2, 1, 4>;   // 256 x 256, 8 waves, ring 136 KB: one workgroup per CU
-using Mid = Shape<1, 4, 4, 1, 1, 3>;    // 128 x 128, 4 waves, ring 51 KB: three per CU
+using Mid = Shape<1, 4, 4, 1, 1, 3>;    // 128 x 128, 4 waves, ring 51 KB: two per CU
 using Low = Shape<1, 2, 2, 2, 2, 3>;    // 64 x 128, 4 waves, ring 75 KB: two per CU
 using Small = Shape<1, 1, 2, 2, 2, 4>;  // 64 x 64, 4 waves, ring 68 KB: two per CU
 
