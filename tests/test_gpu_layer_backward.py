@@ -1,5 +1,5 @@
 """The backward of a group without a concatenated Wᵀ (gate|up and down outside the fused MLP: fused_linear._plain_backward)
-bit for bit against the operations it stands for (/root/reference/scripts/fused_linear.py:128-196): every layer's MX
+bit for bit against the operations it stands for (fused_linear.py:128-196): every layer's MX
 dgrad added in bf16, then dS·S onto that sum; d(xa) and dB as bf16 products, scaled in bf16.  The order matters in the
 last bits: with dS·S added to the last layer's product before the sum over the layers, dx is 3e-3 off (normwise), and a
 dB that is not rounded to bf16 1.7e-3."""
